@@ -181,6 +181,7 @@ def log(msg: str) -> None:
 
 KERNEL_SOURCES = (
     "tropnn_amd/csrc/forward.hip",
+    "tropnn_amd/csrc/gather.hip",
     "tropnn_amd/csrc/backward.hip",
     "tropnn_amd/csrc/device.hpp",
     "tropnn_amd/csrc/launch.hpp",

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define TROPNN_HIP_ABI_VERSION 11
+#define TROPNN_HIP_ABI_VERSION 12
 
 /* status codes */
 #define TROPNN_OK 0
@@ -121,6 +121,26 @@ int tropnn_hip_pairwise_forward(int64_t items, int64_t in_features, int64_t out_
                                 const float *thresholds, const void *lut, int lut_dtype, float output_scale,
                                 float *output, tropnn_route_record *route_record, int64_t *indices, float *margins,
                                 uint8_t *codes, tropnn_stream_t stream);
+
+/*
+ * The same forward with device memory lent for its intermediate codes: the
+ * large-batch kernels then route first (every item's LUT row codes go to the
+ * workspace) and sum the rows out of LDS, each LUT row read once per
+ * workgroup. Same arguments and results as tropnn_hip_pairwise_forward (with
+ * an f16 LUT of 32 MiB or more, outputs agree to f32 rounding: another order of
+ * the sum over tables). workspace: 16-byte aligned device memory of at least
+ * tropnn_hip_pairwise_forward_workspace_size() bytes, or NULL for the plain
+ * forward; written and read by this call's kernels only. The size is 0 for
+ * shapes that take no workspace (and, with an error message, for invalid
+ * arguments). No counterpart in the reference.
+ */
+size_t tropnn_hip_pairwise_forward_workspace_size(int64_t items, int64_t in_features, int64_t out_features,
+                                                  int64_t tables, int64_t comparisons, int lut_dtype);
+int tropnn_hip_pairwise_forward_ws(int64_t items, int64_t in_features, int64_t out_features, int64_t tables,
+                                   int64_t comparisons, const float *latent, const int64_t *anchors,
+                                   const float *thresholds, const void *lut, int lut_dtype, float output_scale,
+                                   float *output, tropnn_route_record *route_record, int64_t *indices, float *margins,
+                                   uint8_t *codes, void *workspace, size_t workspace_bytes, tropnn_stream_t stream);
 
 /*
  * Route only: the comparator codes and margins of every (item, table), with
@@ -259,11 +279,10 @@ int tropnn_hip_cross_entropy(int64_t rows, int64_t classes, const float *logits,
  * calls, tools/benchmarking/benchmark.py:91-118). Arms two caller-created
  * hipEvent_t handles to be recorded on the launch stream immediately before
  * and after the NEXT launch of one kernel:
- *   TROPNN_KERNEL_FORWARD           the fused route + gather + scale kernel (large training
- *                                   shapes: the streamed gather + scale kernel)
- *   TROPNN_KERNEL_FORWARD_ROUTE     the route-record kernel before the streamed gather (training
- *                                   forward with at least 4096 items, LUT rows of whole 128-byte
- *                                   chunks, comparisons <= 8 and a LUT of at least 32 MiB)
+ *   TROPNN_KERNEL_FORWARD           the fused route + gather + scale kernel, or the gather + scale
+ *                                   kernel after a route kernel (with a forward workspace; training
+ *                                   forwards of at least 4096 items over a LUT of at least 32 MiB)
+ *   TROPNN_KERNEL_FORWARD_ROUTE     that route kernel
  *   TROPNN_KERNEL_BACKWARD_TABLE    the per-(table, column chunk) LUT-gradient kernel (with the
  *                                   min-margin STE: also each chunk's partial STE dots)
  *   TROPNN_KERNEL_BACKWARD_ITEM     the per-item STE-dot / input-gradient kernel of the full STE

@@ -288,3 +288,27 @@ def test_autograd_operator_loads_and_binds(lib):
     with pytest.raises(ValueError, match="input-gradient"):
         op(x, anchors, torch.zeros(3, 2), torch.zeros(3, 4, 5), torch.zeros(3, 4, 5), None, None,
            True, True, 0, 1.0, 0, 3)
+
+
+def test_forward_workspace(lib):
+    """The staged forward's workspace: none for small batches, one byte per
+    (item, padded table) where the shape takes it; too small a workspace is
+    refused before any launch, and none means the plain forward."""
+    ws = lib.tropnn_hip_pairwise_forward_workspace_size
+    assert ws(512, 128, 128, 136, 6, ph.LUT_F32) == 0  # latency bound: one launch
+    assert ws(0, 128, 128, 136, 6, ph.LUT_F32) == 0
+    assert ws(8192, 128, 128, 136, 6, ph.LUT_F32) == 0  # below the line of the slice gather's rule
+    assert ws(16384, 128, 128, 136, 6, ph.LUT_F32) == 9 * 16 * 16384  # slice gather: nine blocks of 16 tables
+    assert ws(8195, 300, 250, 100, 5, ph.LUT_F32) == 7 * 16 * 8208  # blocks of 15 in 16 bytes; items rounded up to 16
+    assert ws(8192, 128, 128, 136, 6, ph.LUT_F16) == 0  # the wave-item kernel's rows: not enough to gain
+    assert ws(4096, 1024, 4096, 512, 8, ph.LUT_F16) == 32 * 16 * 4096  # stream gather
+    assert ws(512, 1024, 4096, 512, 8, ph.LUT_F16) == 0  # too few items for the LUT to stream
+    assert ws(8192, 20000, 128, 136, 6, ph.LUT_F32) == 0  # input rows beyond a workgroup's LDS
+    assert ws(8192, 128, 128, 136, 9, ph.LUT_F32) == 0 and "comparisons" in _err(lib)
+    fwd = lib.tropnn_hip_pairwise_forward_ws
+    args = [16384, 128, 128, 136, 6, 16, 16, 16, 16, 0, 1.0, 16, None, None, None, None, 16, 9 * 16 * 16384 - 1, None]
+    assert fwd(*args) == 1 and "workspace" in _err(lib)
+    args[16], args[17] = 24, 1 << 30
+    assert fwd(*args) == 1 and "16-byte" in _err(lib)
+    args[3] = 0
+    assert fwd(*args) == 1 and "tables" in _err(lib)

@@ -26,7 +26,7 @@ from typing import Any
 import torch
 from torch import Tensor
 
-ABI_VERSION = 11
+ABI_VERSION = 12
 LUT_F32, LUT_F16 = 0, 1
 SURROGATE_IDS = {"fast_sigmoid_odd": 0, "izhikevich": 1}
 STE_MIN_MARGIN, STE_FULL = 0, 1
@@ -60,6 +60,8 @@ EXPORTED_SYMBOLS = (
     "tropnn_hip_lut_forward_batch_f32",
     "tropnn_hip_lut_forward_batch_f16",
     "tropnn_hip_pairwise_forward",
+    "tropnn_hip_pairwise_forward_workspace_size",
+    "tropnn_hip_pairwise_forward_ws",
     "tropnn_hip_pairwise_route",
     "tropnn_hip_pairwise_backward_workspace_size",
     "tropnn_hip_pairwise_backward",
@@ -99,6 +101,10 @@ def _declare(lib: ctypes.CDLL) -> None:
         fn.restype = i
     lib.tropnn_hip_pairwise_forward.argtypes = [i64, i64, i64, i64, i64, p, p, p, p, i, f, p, p, p, p, p, p]
     lib.tropnn_hip_pairwise_forward.restype = i
+    lib.tropnn_hip_pairwise_forward_workspace_size.argtypes = [i64, i64, i64, i64, i64, i]
+    lib.tropnn_hip_pairwise_forward_workspace_size.restype = sz
+    lib.tropnn_hip_pairwise_forward_ws.argtypes = [i64, i64, i64, i64, i64, p, p, p, p, i, f, p, p, p, p, p, p, sz, p]
+    lib.tropnn_hip_pairwise_forward_ws.restype = i
     lib.tropnn_hip_pairwise_route.argtypes = [i64, i64, i64, i64, p, p, p, p, p, p, p]
     lib.tropnn_hip_pairwise_route.restype = i
     lib.tropnn_hip_pairwise_backward_workspace_size.argtypes = [i64, i64, i64, i64, i64, i, i]
@@ -182,6 +188,8 @@ def _pairwise_op() -> Any:
             addr("tropnn_hip_pairwise_backward_workspace_size"),
             addr("tropnn_hip_last_error"),
             lib.tropnn_hip_abi_version(),
+            addr("tropnn_hip_pairwise_forward_ws"),
+            addr("tropnn_hip_pairwise_forward_workspace_size"),
         )
         _PAIRWISE_OP = torch.ops.tropnn_hip.pairwise.default
     return _PAIRWISE_OP

@@ -219,11 +219,30 @@ int tropnn_hip_abi_version(void) { return TROPNN_HIP_ABI_VERSION; }
 
 const char *tropnn_hip_last_error(void) { return g_last_error.c_str(); }
 
+size_t tropnn_hip_pairwise_forward_workspace_size(int64_t items, int64_t in_features, int64_t out_features,
+                                                  int64_t tables, int64_t comparisons, int lut_dtype) {
+    tropnn::Dims d{};
+    if (make_dims(items, in_features, out_features, tables, comparisons, lut_dtype, d) != TROPNN_OK) return 0;
+    ok();
+    const tropnn::GatherPlan g = tropnn::plan_gather(d);
+    return g.ok ? g.workspace_bytes : 0;
+}
+
 int tropnn_hip_pairwise_forward(int64_t items, int64_t in_features, int64_t out_features, int64_t tables,
                                 int64_t comparisons, const float *latent, const int64_t *anchors,
                                 const float *thresholds, const void *lut, int lut_dtype, float output_scale,
                                 float *output, tropnn_route_record *route_record, int64_t *indices, float *margins,
                                 uint8_t *codes, tropnn_stream_t stream) {
+    return tropnn_hip_pairwise_forward_ws(items, in_features, out_features, tables, comparisons, latent, anchors,
+                                          thresholds, lut, lut_dtype, output_scale, output, route_record, indices,
+                                          margins, codes, nullptr, 0, stream);
+}
+
+int tropnn_hip_pairwise_forward_ws(int64_t items, int64_t in_features, int64_t out_features, int64_t tables,
+                                   int64_t comparisons, const float *latent, const int64_t *anchors,
+                                   const float *thresholds, const void *lut, int lut_dtype, float output_scale,
+                                   float *output, tropnn_route_record *route_record, int64_t *indices, float *margins,
+                                   uint8_t *codes, void *workspace, size_t workspace_bytes, tropnn_stream_t stream) {
     tropnn::Dims d{};
     if (int rc = make_dims(items, in_features, out_features, tables, comparisons, lut_dtype, d)) return rc;
     // a LUT or output off a 16-byte boundary (a view with a storage offset)
@@ -242,7 +261,26 @@ int tropnn_hip_pairwise_forward(int64_t items, int64_t in_features, int64_t out_
     if (lut_bytes > (int64_t{1} << 31))
         return fail(TROPNN_ERR_UNSUPPORTED, "LUT of %lld bytes exceeds the forward's 2 GiB limit",
                     (long long)lut_bytes);
-    hipError_t e = tropnn::launch_forward(d, p, latent, anchors, thresholds, lut, output_scale, output, route_record,
+    hipError_t e = hipSuccess;
+    if (workspace != nullptr) {
+        const tropnn::GatherPlan g = tropnn::plan_gather(d);
+        const bool rows16 = !misaligned(lut, 16) && !misaligned(output, 16);
+        // the stream gather moves whole 16-byte pieces; a training forward over
+        // a large f32 LUT is left to the streamed kernel of forward.hip
+        if (g.ok && (g.stream ? rows16 : !(route_record && p.stream_ok))) {
+            if (workspace_bytes < g.workspace_bytes)
+                return fail(TROPNN_ERR_INVALID_ARGUMENT, "forward workspace of %zu bytes required, got %zu",
+                            g.workspace_bytes, workspace_bytes);
+            if (misaligned(workspace, 16))
+                return fail(TROPNN_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
+            e = tropnn::launch_gather(d, g, latent, anchors, thresholds, lut, output_scale, output, route_record,
+                                      indices, margins, codes, static_cast<uint32_t *>(workspace),
+                                      static_cast<hipStream_t>(stream));
+            if (e != hipSuccess) return hip_fail("pairwise forward launch", e);
+            return ok();
+        }
+    }
+    e = tropnn::launch_forward(d, p, latent, anchors, thresholds, lut, output_scale, output, route_record,
                                           indices, margins, codes, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail("pairwise forward launch", e);
     return ok();

@@ -38,13 +38,17 @@ struct Abi {
     decltype(&tropnn_hip_pairwise_backward) backward = nullptr;
     decltype(&tropnn_hip_pairwise_backward_workspace_size) workspace_size = nullptr;
     decltype(&tropnn_hip_last_error) last_error = nullptr;
+    decltype(&tropnn_hip_pairwise_forward_ws) forward_ws = nullptr;
+    decltype(&tropnn_hip_pairwise_forward_workspace_size) forward_workspace_size = nullptr;
 };
 Abi g_abi;
 std::atomic<bool> g_bound{false};
 
 // The Python package passes the addresses of the entry points of the
 // libtropnn_hip.so it loaded (ctypes), with that library's ABI version.
-void bind_abi(int64_t forward, int64_t backward, int64_t workspace_size, int64_t last_error, int64_t abi_version) {
+// (forward_ws and forward_workspace_size 0: every forward without a workspace.)
+void bind_abi(int64_t forward, int64_t backward, int64_t workspace_size, int64_t last_error, int64_t abi_version,
+              int64_t forward_ws, int64_t forward_workspace_size) {
     TORCH_CHECK(abi_version == TROPNN_HIP_ABI_VERSION, "libtropnn_hip.so has ABI version ", abi_version,
                 ", the autograd operator was built for ", TROPNN_HIP_ABI_VERSION);
     TORCH_CHECK(forward != 0 && backward != 0 && workspace_size != 0 && last_error != 0,
@@ -53,6 +57,10 @@ void bind_abi(int64_t forward, int64_t backward, int64_t workspace_size, int64_t
     g_abi.backward = reinterpret_cast<decltype(g_abi.backward)>(static_cast<intptr_t>(backward));
     g_abi.workspace_size = reinterpret_cast<decltype(g_abi.workspace_size)>(static_cast<intptr_t>(workspace_size));
     g_abi.last_error = reinterpret_cast<decltype(g_abi.last_error)>(static_cast<intptr_t>(last_error));
+    const bool ws = forward_ws != 0 && forward_workspace_size != 0;
+    g_abi.forward_ws = ws ? reinterpret_cast<decltype(g_abi.forward_ws)>(static_cast<intptr_t>(forward_ws)) : nullptr;
+    g_abi.forward_workspace_size =
+        reinterpret_cast<decltype(g_abi.forward_workspace_size)>(static_cast<intptr_t>(ws ? forward_workspace_size : 0));
     g_bound.store(true, std::memory_order_release);
 }
 
@@ -146,15 +154,27 @@ Forward run_forward(const Dims &d, const Tensor &latent, const Tensor &anchors, 
 
     TORCH_CHECK(g_bound.load(std::memory_order_acquire), "tropnn_hip.pairwise: the C ABI is not bound");
     const int lut_dtype = lut_c.scalar_type() == at::kHalf ? TROPNN_LUT_F16 : TROPNN_LUT_F32;
-    const int rc = g_abi.forward(
-        items, d.in_f, d.out_f, d.tables, d.comps, x.const_data_ptr<float>(), anc.const_data_ptr<int64_t>(),
-        thr.const_data_ptr<float>(), lut_c.const_data_ptr(), lut_dtype, static_cast<float>(output_scale),
-        f.out.mutable_data_ptr<float>(),
-        want_record ? reinterpret_cast<tropnn_route_record *>(f.record.mutable_data_ptr()) : nullptr,
-        full_route ? f.indices.mutable_data_ptr<int64_t>() : nullptr,
-        full_route ? f.margins.mutable_data_ptr<float>()
-                   : (want_margins ? f.saved_margins.mutable_data_ptr<float>() : nullptr),
-        route_mode == kRouteCodes ? f.indices.mutable_data_ptr<uint8_t>() : nullptr, current_stream(x));
+    // large batches route into a workspace first (of this stream, as every
+    // tensor here; the allocator may hand it out again to later work on it)
+    const size_t ws_bytes = g_abi.forward_ws != nullptr ? g_abi.forward_workspace_size(items, d.in_f, d.out_f, d.tables,
+                                                                                      d.comps, lut_dtype)
+                                                        : 0;
+    const Tensor ws = ws_bytes > 0 ? at::empty({static_cast<int64_t>(ws_bytes)}, f32.dtype(at::kByte)) : Tensor();
+    auto *record = want_record ? reinterpret_cast<tropnn_route_record *>(f.record.mutable_data_ptr()) : nullptr;
+    int64_t *indices = full_route ? f.indices.mutable_data_ptr<int64_t>() : nullptr;
+    float *margins = full_route ? f.margins.mutable_data_ptr<float>()
+                                : (want_margins ? f.saved_margins.mutable_data_ptr<float>() : nullptr);
+    uint8_t *codes = route_mode == kRouteCodes ? f.indices.mutable_data_ptr<uint8_t>() : nullptr;
+    const int rc =
+        ws_bytes > 0
+            ? g_abi.forward_ws(items, d.in_f, d.out_f, d.tables, d.comps, x.const_data_ptr<float>(),
+                               anc.const_data_ptr<int64_t>(), thr.const_data_ptr<float>(), lut_c.const_data_ptr(),
+                               lut_dtype, static_cast<float>(output_scale), f.out.mutable_data_ptr<float>(), record,
+                               indices, margins, codes, ws.mutable_data_ptr(), ws_bytes, current_stream(x))
+            : g_abi.forward(items, d.in_f, d.out_f, d.tables, d.comps, x.const_data_ptr<float>(),
+                            anc.const_data_ptr<int64_t>(), thr.const_data_ptr<float>(), lut_c.const_data_ptr(),
+                            lut_dtype, static_cast<float>(output_scale), f.out.mutable_data_ptr<float>(), record,
+                            indices, margins, codes, current_stream(x));
     check_rc(rc, "tropnn_hip_pairwise_forward");
     return f;
 }
@@ -285,7 +305,8 @@ std::tuple<Tensor, Tensor, Tensor> pairwise(const Tensor &latent, const Tensor &
 }  // namespace
 
 TORCH_LIBRARY(tropnn_hip, m) {
-    m.def("bind_abi(int forward, int backward, int workspace_size, int last_error, int abi_version) -> ()",
+    m.def("bind_abi(int forward, int backward, int workspace_size, int last_error, int abi_version, "
+          "int forward_ws=0, int forward_workspace_size=0) -> ()",
           &bind_abi);
     m.def("pairwise(Tensor latent, Tensor anchors, Tensor thresholds, Tensor lut, Tensor lut_read, "
           "Tensor? index_offsets, Tensor? index_entries, bool ste, bool min_margin, int surrogate, "

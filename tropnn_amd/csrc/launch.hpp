@@ -138,6 +138,24 @@ constexpr int item_wave_tables(int esize, int vec) {
 // optionally with one TROPNN_BWD_INPUT_GRAD_* flag (fused path's item role).
 BackwardPlan plan_backward(const Dims &d, int ste_mode);
 
+// Launch shape of the staged forward (gather.hip): a route kernel writes code
+// words to the caller's workspace, then a gather kernel sums the rows.
+struct GatherPlan {
+    bool ok;                 // the shape takes it (given workspace_bytes)
+    bool stream;             // stream gather, else slice gather
+    int per, groups, pitch;  // tables per summed block; code words per item; items of a row of words
+    int quads, route_lds;    // route kernel: groups of four items per workgroup
+    bool route_rec_stage;
+    int wgs, threads, lds_bytes;
+    int blocks, slices, block_items, stage_blocks, stages, zero_off, slice_ipt;
+    int stream_ipt, stream_nblk, stream_gs, stream_stages;
+    size_t workspace_bytes;
+};
+GatherPlan plan_gather(const Dims &d);
+hipError_t launch_gather(const Dims &d, const GatherPlan &p, const float *x, const int64_t *anchors, const float *thr,
+                         const void *lut, float scale, float *out, tropnn_route_record *rec, int64_t *indices,
+                         float *margins, uint8_t *codes, uint32_t *words, hipStream_t stream);
+
 hipError_t launch_forward(const Dims &d, const ForwardPlan &p, const float *x, const int64_t *anchors,
                           const float *thr, const void *lut, float scale, float *out, tropnn_route_record *rec,
                           int64_t *indices, float *margins, uint8_t *codes, hipStream_t stream);
