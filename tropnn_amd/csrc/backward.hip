@@ -76,7 +76,7 @@
 namespace tropnn {
 namespace {
 
-constexpr int kSortThreads = 1024;  // items per tile of the sort kernel
+constexpr int kSortThreads = 1024;  // threads of a sort-kernel workgroup
 constexpr int kRowsThreads = 1024;  // threads of a row-kernel workgroup (but see rows_threads)
 constexpr int kRowsBatch = 8;       // sorted slots per row-kernel batch; rows are padded to whole batches
 
@@ -132,6 +132,7 @@ struct SortArgs {
     int items, out_f, comps, rows, slots;
     int chunk_cols, chunk_vec, chunks;  // P, the row kernel's V, ceil(O / P)
     int batch;                          // rows_batch(V): rows are padded to whole batches
+    int copy_wgs;                       // workgroups before the table ones that copy G (0 without a sort)
 };
 
 // Row kernel (general path), one workgroup per (table, column chunk).
@@ -420,39 +421,75 @@ __device__ void wave_exclusive_scan(int *v, int n, int lane) {
     if (lane == 0) v[n] = carry;
 }
 
-// Counting-sort step of one wave over its 64 items: zeroes the wave's code
-// counts, gives each valid item its rank among the equal codes of the wave
-// (one ballot per code bit) and has each code's first item write the code's
-// count. One wave's LDS operations complete in order, so the zeroing lands
-// before the counts.
-__device__ __forceinline__ int wave_code_rank(int code, bool valid, int R, int C, int *cnt_w, int lane) {
-    for (int k = lane; k < R; k += kWave) cnt_w[k] = 0;
-    uint64_t same = __ballot(valid);
-    for (int c = 0; c < C; ++c) {
-        const uint64_t bc = __ballot(valid && ((code >> c) & 1));
-        same &= ((code >> c) & 1) ? bc : ~bc;
-    }
-    const int rank = __popcll(same & ((1ull << lane) - 1ull));
-    if (valid && rank == 0) cnt_w[code] = __popcll(same);
-    return rank;
+// Sort kernel: the stable counting sort of table t's items by LUT row code,
+// written once for every column chunk of the row kernel. The workgroups before
+// the table ones copy G chunk-major for the row kernel (G's rows are O * 4
+// bytes apart, a power of two at c4, so one column chunk of every row maps
+// onto few L2 sets; the copy makes a chunk one contiguous block): the copy
+// moves at memory rate beside the sort's round trips.
+//   A table's items go in blocks of kSortItems, kSortRounds a thread, all
+// loaded before the first is ranked; a wave takes consecutive items, 64 a
+// round. One ballot per code bit gives an item the mask of equal codes in its
+// round; its rank in the wave is that mask's count below it plus the wave's
+// count of the code so far, which each round's first item of a code carries
+// forward in the wave's own LDS counts (no barrier). The row starts are the
+// counts rounded up to whole batches of rows_batch(V) slots, exclusively
+// scanned; every item goes to its row's start + the waves' counts before its
+// own + its rank (blocks, waves and rounds in order: item order is kept inside
+// a row) as its byte offset b * P * 4 inside a chunk of the copy, with the
+// item's min-margin comparison r, or its neighbour row, in the low bits;
+// padding slots get kSlotPad. One block (8192 items) is read and ranked once;
+// more are counted first, then ranked again as they are placed.
+//   With the full STE it also sums the threshold gradient: -gu of every
+// comparison, a thread's items in order, a fixed tree per wave, waves in order.
+constexpr int kSortRounds = 8;
+constexpr int kSortItems = kSortRounds * kSortThreads;
+constexpr int kCopyWgs = 256;  // copy workgroups, at most
+
+__device__ __forceinline__ void copy_chunked(const SortArgs &a, int w, int wgs) {
+    // rows (chunk, item) of P columns, a contiguous range of them per
+    // workgroup; the row's pieces of V columns go to consecutive threads, so
+    // both sides are contiguous. Pieces past O stay unwritten (the row kernel
+    // masks those columns).
+    const int piece_cols = a.chunk_vec >= 4 ? 4 : a.chunk_vec;
+    const int pieces = a.chunk_cols / piece_cols, log2p = 31 - __builtin_clz(pieces);  // a power of two
+    const int64_t total = static_cast<int64_t>(a.chunks) * a.items;
+    const int r0 = static_cast<int>(total * w / wgs), r1 = static_cast<int>(total * (w + 1) / wgs);
+    const int n = (r1 - r0) << log2p;
+    constexpr int kU = 4;  // pieces in flight per thread
+    auto each = [&](auto vec) {
+        using V = decltype(vec);
+        for (int k0 = threadIdx.x; k0 < n; k0 += kU * kSortThreads) {
+            V v[kU];
+            int dst[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const int k = k0 + u * kSortThreads, cb = r0 + (k >> log2p), piece = k & (pieces - 1);
+                const int chunk = cb / a.items, b = cb - chunk * a.items, col = chunk * a.chunk_cols + piece * piece_cols;
+                dst[u] = k < n && col < a.out_f ? piece : -1;
+                if (dst[u] >= 0) v[u] = *reinterpret_cast<const V *>(a.grad_out + static_cast<size_t>(b) * a.out_f + col);
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (dst[u] >= 0)
+                    *reinterpret_cast<V *>(a.g_chunked + static_cast<size_t>(r0 + ((k0 + u * kSortThreads) >> log2p)) * a.chunk_cols +
+                                           dst[u] * piece_cols) = v[u];
+        }
+    };
+    if (piece_cols == 4)
+        each(vec_t<float, 4>{});
+    else if (piece_cols == 2)
+        each(vec_t<float, 2>{});
+    else
+        each(0.f);
 }
 
-// Sort kernel: the stable counting sort of table t's items by LUT row code,
-// written once for every column chunk of the row kernel, and table t's share
-// of a chunk-major copy of G for the row kernel (G's rows are O * 4 bytes
-// apart, a power of two at c4, so one column chunk of every row maps onto
-// few L2 sets; the copy makes a chunk one contiguous block). Pass 1 counts each
-// code over tiles of 1024 items (and sums the threshold gradient's partials:
-// -gu at each item's min-margin comparison, or at every comparison with the
-// full STE, a fixed tree per wave, waves in order, tiles in order); the row
-// starts are the counts rounded up to whole batches of rows_batch(V) slots,
-// exclusively scanned. Pass 2 places every item at its row's next free slot
-// (tiles, waves and lanes in order, so item order is kept inside a row) as
-// its byte offset b * P * 4 inside a chunk of the copy, with the item's
-// min-margin comparison r in the offset's low 3 bits (P * 4 >= 16); padding
-// slots get kSlotPad.
 __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArgs a) {
     constexpr int kWaves = kSortThreads / kWave;
+    if (static_cast<int>(blockIdx.x) < a.copy_wgs) {  // copy role (uniform per workgroup)
+        copy_chunked(a, blockIdx.x, a.copy_wgs);
+        return;
+    }
     const int K = a.batch;
     extern __shared__ __align__(16) unsigned char lds[];
     const int R = a.rows, C = a.comps;
@@ -460,43 +497,57 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
     int *base = cnt + kWaves * R;                            // [R] next free slot of each row
     int *wtot = base + R;                                    // [waves] scan carries
     float *tp = reinterpret_cast<float *>(wtot + kWaves);    // [waves][8] threshold partials
-    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int t = blockIdx.x - a.copy_wgs, tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint64_t *rec_t = a.rec + static_cast<size_t>(t) * a.items;
-    const bool thr = a.grad_thr != nullptr;
-    const float *gu_t = thr ? a.gu + static_cast<size_t>(t) * (a.full ? C : 1) * a.items : nullptr;
-    if (lane < 8) tp[wave * 8 + lane] = 0.f;  // each wave its own slots
-
-    // 1. per-code totals, threshold partials
-    int tot = 0;  // thread k < R: items of code k
-    for (int tile0 = 0; tile0 < a.items; tile0 += kSortThreads) {
-        const int b = tile0 + tid;
-        const bool valid = b < a.items;
-        const uint64_t r = valid ? rec_t[b] : 0ull;
-        wave_code_rank(rec_code(r) & (R - 1), valid, R, C, cnt + wave * R, lane);
-        if (thr) {
-            float tv[8];
-            if (a.full) {
-#pragma unroll
-                for (int c = 0; c < 8; ++c) tv[c] = valid && c < C ? -gu_t[static_cast<size_t>(c) * a.items + b] : 0.f;
-            } else {
-                const float gu = valid ? gu_t[b] : 0.f;
-                const int rr = rec_r(r) & 7;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) tv[c] = rr == c ? -gu : 0.f;
-            }
-            const float s = reduce_scatter<kWave, 8>(tv, lane);  // lane 8c: the wave's sum for comparison c
-            if ((lane & 7) == 0) tp[wave * 8 + (lane >> 3)] += s;
-        }
-        __syncthreads();
-        if (tid < R)
-            for (int w = 0; w < kWaves; ++w) tot += cnt[w * R + tid];
-        __syncthreads();
-    }
+    const bool thr = a.grad_thr != nullptr;  // full STE only
 
     if (a.slot_off != nullptr) {
-        // 2. row starts: totals rounded up to whole batches, exclusive scan;
-        //    padding slots and the row of every batch
+        uint32_t hi[kSortRounds];  // route record's code | r << 16
+        int rank[kSortRounds];
+        // block of items from s0: this wave's share is rounds * 64 consecutive items
+        auto load = [&](int s0, int rounds) {
+#pragma unroll
+            for (int j = 0; j < kSortRounds; ++j) {
+                const int b = s0 + (wave * rounds + j) * kWave + lane;
+                hi[j] = j < rounds && b < a.items ? static_cast<uint32_t>(rec_t[b] >> 32) : 0u;
+            }
+        };
+        auto rank_all = [&](int s0, int rounds) {
+            int *cw = cnt + wave * R;
+            for (int k = lane; k < R; k += kWave) cw[k] = 0;
+#pragma unroll
+            for (int j = 0; j < kSortRounds; ++j) {
+                if (j < rounds) {  // uniform
+                    const bool valid = s0 + (wave * rounds + j) * kWave + lane < a.items;
+                    const int code = static_cast<int>(hi[j] & 0xffffu) & (R - 1);
+                    uint64_t same = __ballot(valid);
+                    for (int c = 0; c < C; ++c) {
+                        const uint64_t bc = __ballot(valid && ((code >> c) & 1));
+                        same &= ((code >> c) & 1) ? bc : ~bc;
+                    }
+                    const int below = __popcll(same & ((1ull << lane) - 1ull));
+                    const int prior = cw[code];  // (LDS operations of one wave complete in order)
+                    rank[j] = prior + below;
+                    if (valid && below == 0) cw[code] = prior + __popcll(same);
+                }
+            }
+        };
+        const int blocks = (a.items + kSortItems - 1) / kSortItems;
+        auto rounds_of = [&](int s0) { return (min(kSortItems, a.items - s0) + kSortThreads - 1) / kSortThreads; };
+
+        // 1. totals of every code
+        int tot = 0;  // thread k < R: items of code k
+        for (int q = 0; q < blocks; ++q) {
+            const int s0 = q * kSortItems, rounds = rounds_of(s0);
+            load(s0, rounds);
+            rank_all(s0, rounds);
+            __syncthreads();
+            if (tid < R)
+                for (int w = 0; w < kWaves; ++w) tot += cnt[w * R + tid];
+            if (blocks > 1) __syncthreads();  // the next block rewrites the counts
+        }
+        // 2. row starts: totals rounded up to whole batches, exclusive scan; padding slots
         const int nscan = ((R + kWave - 1) / kWave) * kWave;  // whole waves
         int padded = 0, incl = 0;
         if (tid < nscan) {
@@ -510,70 +561,55 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
                 for (int w = 0; w < wave; ++w) incl += wtot[w];
         }
         uint32_t *so = a.slot_off + static_cast<size_t>(t) * a.slots;
+        int32_t *br = a.batch_row + static_cast<size_t>(t) * (a.slots / K);
+        int run = incl - padded;  // thread k < R: row k's next free slot
         if (tid < R) {
-            const int excl = incl - padded;
-            a.row_start[static_cast<size_t>(t) * (R + 1) + tid] = excl;
+            a.row_start[static_cast<size_t>(t) * (R + 1) + tid] = run;
             if (tid == R - 1) a.row_start[static_cast<size_t>(t) * (R + 1) + R] = incl;
-            base[tid] = excl;
-            for (int q = excl + tot; q < excl + padded; ++q) so[q] = kSlotPad;
-            int32_t *br = a.batch_row + static_cast<size_t>(t) * (a.slots / K);
-            for (int bb = excl / K; bb < incl / K; ++bb) br[bb] = tid;
+            for (int q = run + tot; q < run + padded; ++q) so[q] = kSlotPad;
         }
-        __syncthreads();
-
-        // 3. stable placement
-        for (int tile0 = 0; tile0 < a.items; tile0 += kSortThreads) {
-            const int b = tile0 + tid;
-            const bool valid = b < a.items;
-            const uint64_t rr = valid ? rec_t[b] : 0ull;
-            const int code = rec_code(rr) & (R - 1);
-            const int rank = wave_code_rank(code, valid, R, C, cnt + wave * R, lane);
-            __syncthreads();
-            if (tid < R) {
-                int run = base[tid];
+        // 3. stable placement; a batch's first slot, never a padding one, names the batch's row
+        for (int q = 0; q < blocks; ++q) {
+            const int s0 = q * kSortItems, rounds = rounds_of(s0);
+            if (blocks > 1) {
+                load(s0, rounds);
+                __syncthreads();
+                rank_all(s0, rounds);
+                __syncthreads();
+            }
+            if (tid < R)
                 for (int w = 0; w < kWaves; ++w) {
                     const int x = cnt[w * R + tid];
                     cnt[w * R + tid] = run;
                     run += x;
                 }
-                base[tid] = run;
-            }
             __syncthreads();
-            if (valid) {
-                const int r = rec_r(rr) & 7;
-                const uint32_t low = a.nb_pack ? static_cast<uint32_t>((code ^ (1 << r)) & (R - 1)) : static_cast<uint32_t>(r);
-                so[cnt[wave * R + code] + rank] = (static_cast<uint32_t>(b) * static_cast<uint32_t>(a.chunk_cols) * 4u) | low;
-            }
-            __syncthreads();  // the next tile rewrites the counts
-        }
-
-        // 4. this table's share of the chunk-major copy: rows (chunk, item)
-        //    of P columns, a contiguous range of them per table; the row's
-        //    pieces of V columns go to consecutive threads, so both sides are
-        //    contiguous. Pieces past O stay unwritten (the row kernel masks
-        //    those columns).
-        const int pieces = a.chunk_cols / a.chunk_vec;  // S, a power of two <= 64
-        const int rows_total = a.chunks * a.items;
-        const int r0 = static_cast<int>(static_cast<int64_t>(rows_total) * t / gridDim.x);
-        const int r1 = static_cast<int>(static_cast<int64_t>(rows_total) * (t + 1) / gridDim.x);
-        const int piece = tid % pieces;
-        for (int cb = r0 + tid / pieces; cb < r1; cb += kSortThreads / pieces) {
-            const int chunk = cb / a.items, b = cb - chunk * a.items;
-            const int col = chunk * a.chunk_cols + piece * a.chunk_vec;
-            if (col >= a.out_f) continue;
-            const float *src = a.grad_out + static_cast<size_t>(b) * a.out_f + col;
-            float *dst = a.g_chunked + static_cast<size_t>(cb) * a.chunk_cols + piece * a.chunk_vec;
-            if (a.chunk_vec % 4 == 0) {
-                for (int e = 0; e < a.chunk_vec; e += 4)
-                    *reinterpret_cast<vec_t<float, 4> *>(dst + e) = *reinterpret_cast<const vec_t<float, 4> *>(src + e);
-            } else {
-                for (int e = 0; e < a.chunk_vec; ++e) dst[e] = src[e];
+#pragma unroll
+            for (int j = 0; j < kSortRounds; ++j) {
+                const int b = s0 + (wave * rounds + j) * kWave + lane;
+                if (j < rounds && b < a.items) {
+                    const int code = static_cast<int>(hi[j] & 0xffffu) & (R - 1), r = static_cast<int>(hi[j] >> 16) & 7;
+                    const uint32_t low = a.nb_pack ? static_cast<uint32_t>((code ^ (1 << r)) & (R - 1)) : static_cast<uint32_t>(r);
+                    const int pos = cnt[wave * R + code] + rank[j];
+                    so[pos] = (static_cast<uint32_t>(b) * static_cast<uint32_t>(a.chunk_cols) * 4u) | low;
+                    if ((pos & (K - 1)) == 0) br[pos / K] = code;  // K is 4 or 8
+                }
             }
         }
     }
 
-    // 5. threshold gradient: the waves' sums in wave order
+    // 4. threshold gradient (full STE)
     if (thr) {
+        const float *gu_t = a.gu + static_cast<size_t>(t) * C * a.items;
+        float tv[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) tv[c] = 0.f;
+        for (int b = tid; b < a.items; b += kSortThreads)
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                if (c < C) tv[c] -= gu_t[static_cast<size_t>(c) * a.items + b];
+        const float s = reduce_scatter<kWave, 8>(tv, lane);  // lane 8c: the wave's sum for comparison c
+        if ((lane & 7) == 0) tp[wave * 8 + (lane >> 3)] = s;
         __syncthreads();
         if (tid < C) {
             float sum = tp[tid];
@@ -863,19 +899,19 @@ __global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_ro
     }
 }
 
-// Reduce kernel (general path, min-margin): one workgroup per table, one
-// thread per sorted slot of a tile of 1024 slots. A slot's STE dot is the
-// sum of its chunks' partial dots in chunk order (contiguous reads across the
-// threads); gu = dot * scale * surrogate'(u) with u from the slot item's
-// route record. It stores the {gu, r} record for the scatter kernel and sums
-// the threshold gradient, -gu at the item's min-margin comparison (a fixed
-// tree per wave, waves in order, tiles in order: slots in sorted order).
-// Padding slots carry no gu.
+// Reduce kernel (general path, min-margin): one workgroup per table, kU
+// sorted slots per thread at a time, kReduceThreads apart, so that their round
+// trips overlap. A slot's STE dot is the sum of its chunks' partial dots in
+// chunk order (contiguous reads across the threads); gu = dot * scale *
+// surrogate'(u) with u from the slot item's route record. It stores the
+// {gu, r} record for the scatter kernel and sums the threshold gradient, -gu
+// at the item's min-margin comparison (a thread's slots in order, a fixed tree
+// per wave, waves in order). Padding slots carry no gu.
 constexpr int kReduceThreads = 1024;
 constexpr int kReduceStageBytes = 64 * 1024;  // a table's {gu, r} records staged in LDS up to 8192 items
 
 __global__ __launch_bounds__(kReduceThreads) void pairwise_bwd_reduce_kernel(ReduceArgs a) {
-    constexpr int kWaves = kReduceThreads / kWave;
+    constexpr int kWaves = kReduceThreads / kWave, kU = 4;
     __shared__ float tp[kWaves * 8];
     // with `stage`, the table's {gu, r} records gather in LDS (in item order)
     // and leave as whole lines after the walk, instead of as scattered
@@ -887,42 +923,58 @@ __global__ __launch_bounds__(kReduceThreads) void pairwise_bwd_reduce_kernel(Red
     const uint32_t *so = a.slot_off + static_cast<size_t>(t) * a.slots;
     const float *pd = a.pdot + static_cast<size_t>(t) * a.chunks * a.slots;
     const int n_slots = a.row_start[static_cast<size_t>(t) * (a.rows + 1) + a.rows];
-    if (lane < 8) tp[wave * 8 + lane] = 0.f;  // each wave its own slots
-    for (int q0 = 0; q0 < n_slots; q0 += kReduceThreads) {
-        const int q = q0 + tid;
-        const uint32_t off = q < n_slots ? so[q] : kSlotPad;
-        const bool live = off != kSlotPad;
-        const int b = static_cast<int>(off >> a.item_shift);
-        const uint64_t rr = live ? rec_t[b] : 0ull;
-        float dot = 0.f;
-        if (live) {
-            constexpr int kU = 8;  // partial dots in flight
-            int c = 0;
-            for (; c + kU <= a.chunks; c += kU) {
-                float v[kU];
+    float tv[8];
 #pragma unroll
-                for (int u = 0; u < kU; ++u) v[u] = pd[static_cast<size_t>(c + u) * a.slots + q];
+    for (int c = 0; c < 8; ++c) tv[c] = 0.f;
+    for (int q0 = tid; q0 < n_slots; q0 += kU * kReduceThreads) {
+        uint32_t off[kU];
+        uint64_t rr[kU];
+        float dot[kU];
 #pragma unroll
-                for (int u = 0; u < kU; ++u) dot += v[u];
+        for (int u = 0; u < kU; ++u) off[u] = q0 + u * kReduceThreads < n_slots ? so[q0 + u * kReduceThreads] : kSlotPad;
+#pragma unroll
+        for (int u = 0; u < kU; ++u) dot[u] = 0.f;
+        // the slots' dots, kD chunks of each in flight, summed in chunk order
+        // (a padding slot's dots are loaded and dropped)
+        constexpr int kD = 4;
+        auto sum = [&](int c, auto n) {
+            constexpr int N = decltype(n)::value;
+            float v[N][kU];
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+#pragma unroll
+                for (int u = 0; u < kU; ++u)
+                    v[e][u] = q0 + u * kReduceThreads < n_slots ? pd[static_cast<size_t>(c + e) * a.slots + q0 + u * kReduceThreads] : 0.f;
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+#pragma unroll
+                for (int u = 0; u < kU; ++u) dot[u] += v[e][u];
+        };
+        int c = 0;
+        for (; c + kD <= a.chunks; c += kD) sum(c, std::integral_constant<int, kD>{});
+        for (; c < a.chunks; ++c) sum(c, std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int u = 0; u < kU; ++u) rr[u] = off[u] != kSlotPad ? rec_t[off[u] >> a.item_shift] : 0ull;
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const bool live = off[u] != kSlotPad;
+            const int b = static_cast<int>(off[u] >> a.item_shift);
+            const int r = rec_r(rr[u]) & 7;  // the slot's low bits may hold the neighbour row instead
+            const float gu = live ? dot[u] * a.scale * surrogate_grad(rec_u(rr[u]), a.surrogate) : 0.f;
+            if (live && a.gurec != nullptr) {
+                const uint64_t out = static_cast<uint64_t>(__builtin_bit_cast(uint32_t, gu)) | (static_cast<uint64_t>(r) << 32);
+                if (a.stage)
+                    gstage[b] = out;
+                else
+                    a.gurec[static_cast<size_t>(t) * a.items + b] = out;
             }
-            for (; c < a.chunks; ++c) dot += pd[static_cast<size_t>(c) * a.slots + q];
-        }
-        const int r = rec_r(rr) & 7;  // the slot's low bits may hold the neighbour row instead
-        const float gu = live ? dot * a.scale * surrogate_grad(rec_u(rr), a.surrogate) : 0.f;
-        if (live && a.gurec != nullptr) {
-            const uint64_t out = static_cast<uint64_t>(__builtin_bit_cast(uint32_t, gu)) | (static_cast<uint64_t>(r) << 32);
-            if (a.stage)
-                gstage[b] = out;
-            else
-                a.gurec[static_cast<size_t>(t) * a.items + b] = out;
-        }
-        if (a.grad_thr != nullptr) {
-            float tv[8];
 #pragma unroll
-            for (int c = 0; c < 8; ++c) tv[c] = live && r == c ? -gu : 0.f;
-            const float sum = reduce_scatter<kWave, 8>(tv, lane);  // lane 8c: the wave's sum for comparison c
-            if ((lane & 7) == 0) tp[wave * 8 + (lane >> 3)] += sum;
+            for (int k = 0; k < 8; ++k) tv[k] += live && r == k ? -gu : 0.f;
         }
+    }
+    if (a.grad_thr != nullptr) {
+        const float sum = reduce_scatter<kWave, 8>(tv, lane);  // lane 8c: the wave's sum for comparison c
+        if ((lane & 7) == 0) tp[wave * 8 + (lane >> 3)] = sum;
     }
     if (a.stage || a.grad_thr != nullptr) __syncthreads();
     if (a.stage)  // every item of the table had one live slot
@@ -2230,7 +2282,10 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     so.comps = d.comps;
     so.rows = d.rows;
     so.slots = p.sort_slots;
-    if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_SORT, pairwise_bwd_sort_kernel, dim3(d.tables),
+    // about 64 KB of G per copy workgroup, one to each CU at most
+    const long long copy_bytes = static_cast<long long>(d.items) * d.out_f * 4;
+    so.copy_wgs = so.slot_off == nullptr ? 0 : static_cast<int>(copy_bytes / (64 * 1024) + 1 < kCopyWgs ? copy_bytes / (64 * 1024) + 1 : kCopyWgs);
+    if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_SORT, pairwise_bwd_sort_kernel, dim3(d.tables + so.copy_wgs),
                                      dim3(kSortThreads), p.sort_lds_bytes, stream, so);
         e != hipSuccess || so.slot_off == nullptr)
         return e;
