@@ -1,0 +1,57 @@
+"""The general backward's row kernel when a (table, column chunk)'s sorted
+batches are shared by several workgroups (few tables or chunks, large batches):
+rows of the LUT gradient that cross workgroups are merged from their part sums.
+Against the oracle; with large thresholds most items fall into a few rows, so
+that one row spans several parts, and many rows are empty."""
+from __future__ import annotations
+
+import importlib
+
+import pytest
+import torch
+
+from test_gpu_parity import DEV, F16_TOL, F32_TOL, assert_train_parity, make_pair, rel_err, seeded, train_step
+
+ph = importlib.import_module("tropnn_amd.backends.pairwise_hip")
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize(
+    "i,o,t,c,b,thr_std,lut_dtype",
+    [
+        (64, 320, 9, 6, 4100, 0.3, "f32"),   # 45 units: four parts
+        (64, 320, 2, 3, 8200, 5.0, "f32"),   # eight parts, rows spanning several of them
+        (40, 1000, 1, 1, 8195, 0.3, "f32"),  # two rows, each over half the parts
+        (64, 90, 5, 8, 5000, 4.0, "f16"),    # two columns per lane, 8-slot batches, f16 rows
+        (33, 31, 3, 8, 9000, 0.3, "f32"),    # one column per lane, 1024-thread workgroups
+    ],
+)
+def test_rows_split_over_parts(i, o, t, c, b, thr_std, lut_dtype):
+    ref, hip = make_pair(i, o, t, c, seed=3, thr_std=thr_std, lut_dtype=lut_dtype)
+    x, g = seeded((b, i), seed=1), seeded((b, 1, o), seed=2)
+    # rows of thousands of items: the f32 oracle's own rounding of such sums
+    # reaches 4e-4 of an element (sqrt(8200) eps against a cancelled sum)
+    assert_train_parity(ref, hip, *train_step(ref, hip, x, g), tol=F16_TOL if lut_dtype == "f16" else F32_TOL, elem_rtol=1e-3)
+
+
+def test_allocation_free_backward_keeps_its_range():
+    """A shape whose split plan needs more than the allocation-free entry
+    point's 32 MiB, but whose plain one fits: still served."""
+    b, i, o, t, c = 12000, 32, 512, 16, 6
+    lib = ph.load_library()
+    assert lib.tropnn_hip_pairwise_backward_workspace_size(b, i, o, t, c, ph.LUT_F32, ph.STE_MIN_MARGIN) > 32 << 20
+    _, hip = make_pair(i, o, t, c, seed=3, thr_std=0.3)
+    x, g = seeded((b, i), seed=1).to(DEV).requires_grad_(True), seeded((b, 1, o), seed=2).to(DEV)
+    hip.train()(x).backward(g)
+    _, rec, *_ = ph._route_forward(x.detach().unsqueeze(1), hip.anchors, hip.thresholds.detach(), hip.lut.detach(),
+                                   output_scale=hip.output_scale, want_record=True, return_route=False)
+    offsets, entries = ph.anchor_index(hip.anchors, i)
+    out = [torch.empty(b, i, device=DEV), torch.empty(t, c, device=DEV), torch.empty(t, 1 << c, o, device=DEV)]
+    rc = lib.tropnn_hip_pairwise_backward_noalloc(
+        b, i, o, t, c, g.data_ptr(), hip.lut.data_ptr(), ph.LUT_F32, rec.data_ptr(), None, offsets.data_ptr(),
+        entries.data_ptr(), hip.output_scale, ph.STE_MIN_MARGIN, 0, *(v.data_ptr() for v in out),
+        torch.cuda.current_stream(DEV).cuda_stream)
+    assert rc == 0, lib.tropnn_hip_last_error()
+    for got, want in zip(out, (x.grad, hip.thresholds.grad, hip.lut.grad)):
+        assert rel_err(got.cpu(), want.cpu()) <= 1e-6  # another order of a few row sums

@@ -340,7 +340,7 @@ size_t tropnn_hip_pairwise_backward_workspace_size(int64_t items, int64_t in_fea
     if (make_dims(items, in_features, out_features, tables, comparisons, lut_dtype, d) != TROPNN_OK) return 0;
     if (check_ste_mode(ste_mode) != TROPNN_OK) return 0;
     ok();
-    return tropnn::plan_backward(d, ste_mode).workspace_bytes;
+    return tropnn::plan_backward(d, ste_mode, false).workspace_bytes;
 }
 
 int tropnn_hip_build_anchor_index(int64_t in_features, int64_t tables, int64_t comparisons, const int64_t *anchors,
@@ -359,18 +359,18 @@ int tropnn_hip_build_anchor_index(int64_t in_features, int64_t tables, int64_t c
     return ok();
 }
 
-int tropnn_hip_pairwise_backward(int64_t items, int64_t in_features, int64_t out_features, int64_t tables,
-                                 int64_t comparisons, const float *grad_output, const void *lut, int lut_dtype,
-                                 const tropnn_route_record *route_record, const float *margins,
-                                 const int32_t *index_offsets, const int32_t *index_entries, float output_scale,
-                                 int ste_mode, int surrogate, float *grad_latent, float *grad_thresholds,
-                                 float *grad_lut, void *workspace, size_t workspace_bytes, tropnn_stream_t stream) {
+// The backward; lean: planned for the smallest workspace (see plan_backward).
+static int backward(int64_t items, int64_t in_features, int64_t out_features, int64_t tables, int64_t comparisons,
+                    const float *grad_output, const void *lut, int lut_dtype, const tropnn_route_record *route_record,
+                    const float *margins, const int32_t *index_offsets, const int32_t *index_entries,
+                    float output_scale, int ste_mode, int surrogate, float *grad_latent, float *grad_thresholds,
+                    float *grad_lut, void *workspace, size_t workspace_bytes, bool lean, tropnn_stream_t stream) {
     tropnn::Dims d{};
     if (int rc = make_dims(items, in_features, out_features, tables, comparisons, lut_dtype, d)) return rc;
     if (int rc = check_ste_mode(ste_mode)) return rc;
     if (surrogate != TROPNN_SURROGATE_FAST_SIGMOID_ODD && surrogate != TROPNN_SURROGATE_IZHIKEVICH)
         return fail(TROPNN_ERR_INVALID_ARGUMENT, "surrogate must be a TROPNN_SURROGATE_* value");
-    const tropnn::BackwardPlan p = tropnn::plan_backward(d, ste_mode);
+    const tropnn::BackwardPlan p = tropnn::plan_backward(d, ste_mode, lean);
     if (d.items == 0) {
         // no items: the parameter gradients are zero (a fill kernel, not a
         // memset, so the call stays capturable in a HIP graph)
@@ -428,6 +428,17 @@ int tropnn_hip_pairwise_backward(int64_t items, int64_t in_features, int64_t out
     return ok();
 }
 
+int tropnn_hip_pairwise_backward(int64_t items, int64_t in_features, int64_t out_features, int64_t tables,
+                                 int64_t comparisons, const float *grad_output, const void *lut, int lut_dtype,
+                                 const tropnn_route_record *route_record, const float *margins,
+                                 const int32_t *index_offsets, const int32_t *index_entries, float output_scale,
+                                 int ste_mode, int surrogate, float *grad_latent, float *grad_thresholds,
+                                 float *grad_lut, void *workspace, size_t workspace_bytes, tropnn_stream_t stream) {
+    return backward(items, in_features, out_features, tables, comparisons, grad_output, lut, lut_dtype, route_record,
+                    margins, index_offsets, index_entries, output_scale, ste_mode, surrogate, grad_latent,
+                    grad_thresholds, grad_lut, workspace, workspace_bytes, false, stream);
+}
+
 int tropnn_hip_pairwise_backward_noalloc(int64_t items, int64_t in_features, int64_t out_features, int64_t tables,
                                          int64_t comparisons, const float *grad_output, const void *lut,
                                          int lut_dtype, const tropnn_route_record *route_record, const float *margins,
@@ -437,7 +448,9 @@ int tropnn_hip_pairwise_backward_noalloc(int64_t items, int64_t in_features, int
     tropnn::Dims d{};
     if (int rc = make_dims(items, in_features, out_features, tables, comparisons, lut_dtype, d)) return rc;
     if (int rc = check_ste_mode(ste_mode)) return rc;
-    const size_t need = tropnn::plan_backward(d, ste_mode).workspace_bytes;
+    size_t need = tropnn::plan_backward(d, ste_mode, false).workspace_bytes;
+    const bool lean = need > sizeof scratch;  // the backward that keeps less before none at all
+    if (lean) need = tropnn::plan_backward(d, ste_mode, true).workspace_bytes;
     if (need > sizeof scratch)
         return fail(TROPNN_ERR_UNSUPPORTED,
                     "this backward needs %zu bytes of workspace, over the %zu bytes of the allocation-free entry "
@@ -447,10 +460,9 @@ int tropnn_hip_pairwise_backward_noalloc(int64_t items, int64_t in_features, int
     if (d.items > 0 && (grad_latent || grad_thresholds || grad_lut)) {
         if (int rc = scratch_for_stream(static_cast<hipStream_t>(stream), &ws)) return rc;
     }
-    return tropnn_hip_pairwise_backward(items, in_features, out_features, tables, comparisons, grad_output, lut,
-                                        lut_dtype, route_record, margins, index_offsets, index_entries, output_scale,
-                                        ste_mode, surrogate, grad_latent, grad_thresholds, grad_lut, ws,
-                                        ws != nullptr ? sizeof scratch : 0, stream);
+    return backward(items, in_features, out_features, tables, comparisons, grad_output, lut, lut_dtype, route_record,
+                    margins, index_offsets, index_entries, output_scale, ste_mode, surrogate, grad_latent,
+                    grad_thresholds, grad_lut, ws, ws != nullptr ? sizeof scratch : 0, lean, stream);
 }
 
 }  // extern "C"

@@ -77,7 +77,7 @@ namespace tropnn {
 namespace {
 
 constexpr int kSortThreads = 1024;  // threads of a sort-kernel workgroup
-constexpr int kRowsThreads = 1024;  // threads of a row-kernel workgroup (but see rows_threads)
+constexpr int kRowsThreads = 1024;  // threads of a row-kernel workgroup at most
 constexpr int kRowsBatch = 8;       // sorted slots per row-kernel batch; rows are padded to whole batches
 
 // A row-kernel batch: 32 grad-row floats per lane in flight, so 4 slots for
@@ -85,19 +85,20 @@ constexpr int kRowsBatch = 8;       // sorted slots per row-kernel batch; rows a
 // batches of this size.
 constexpr int rows_batch(int vec) { return vec == 8 ? 4 : kRowsBatch; }
 
-// Threads of a row-kernel workgroup. With partial dots over an f16 LUT the
-// LUT chunk stays f16 in LDS (32 KB at 64 columns), so that a 512-thread
-// workgroup needs under 80 KB and two share a CU: one's staging and combine
-// overlap the other's walk. Otherwise 1024.
-constexpr int rows_threads(bool dots, int lut_esize) { return dots && lut_esize == 2 ? 512 : kRowsThreads; }
+// Threads of a row-kernel workgroup: 512 with partial dots where two such
+// workgroups fit a CU's LDS, so that one's staging and combine overlap the
+// other's walk (the LUT chunk in its element type, 32 KB at 64 columns and 256
+// f16 rows), else 1024.
+constexpr int kRowsSmall = 512;
+constexpr int kRowsMaxParts = 16;
+constexpr int kCus = 256;  // gfx950 (MI355X)
+constexpr int kRowsSmallLds = 78 * 1024;
 // Whether the row kernel with nb packed in its slot offsets forms the
 // neighbour row's LDS address with one byte permute: the LUT chunk held in
-// LDS (f32 in 1024-thread workgroups, else f16) has rows of 256 bytes. The
-// permute yields the address relative to the chunk, so the chunk must sit at
-// LDS address 0; launch_rows_vs checks that on the host.
-constexpr bool rows_nb_perm(bool dots, int lut_esize, int s, int v) {
-    return dots && s * v * (rows_threads(dots, lut_esize) == kRowsThreads ? 4 : 2) == 256;
-}
+// LDS has rows of 256 bytes. The permute yields the address relative to the
+// chunk, so the chunk must sit at LDS address 0; launch_rows_vs checks that on
+// the host.
+constexpr bool rows_nb_perm(bool dots, int lut_esize, int s, int v) { return dots && s * v * lut_esize == 256; }
 constexpr int kRowsChunk = 64;     // columns of a row-kernel workgroup (at most): 2 MB of G at c4, within an L2
 constexpr uint32_t kSlotPad = 0x80000000u;  // grad-row offset of a padding slot: past any grad buffer (<= 2 GiB)
 constexpr int kEntries = 16;       // index entries a walker reads per batch
@@ -152,6 +153,8 @@ struct RowsArgs {
     float *pdot;           // [T][chunks][slots] per sorted slot: sum over the chunk's columns of G (L[nb] - L[code]), unscaled
     int items, chunks, lut_off, rs_off;  // LDS byte offsets: LUT chunk (0 with dots), row starts
     int ring_off;                        // LDS byte offset of the row groups' slot-offset rings
+    int parts;                           // workgroups that share a (table, chunk)'s batches
+    float *part_sums;                    // [T][chunks][parts][2][P] sums of the rows that cross parts
 };
 
 // Reduce kernel (general path, min-margin), one workgroup per table.
@@ -167,6 +170,10 @@ struct ReduceArgs {
     int items, chunks, comps, rows, slots;
     int item_shift;        // slot offset >> item_shift = item (offsets are item * P * 4)
     int stage;             // gurec's records of a table gathered in LDS first (items * 8 bytes of dynamic LDS)
+    // rows split over the row kernel's parts (parts > 1, grad_lut asked for)
+    const float *part_sums;  // [T][chunks][parts][2][P]
+    float *grad_lut;
+    int tables, parts, groups, batch, out_f, chunk_cols;  // groups: row groups of a part
 };
 
 __device__ __forceinline__ int rec_code(uint64_t r) { return static_cast<int>((r >> 32) & 0xffffu); }
@@ -642,9 +649,8 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
 // row crossing the range's start (end) leaves its sum in the group's slot 0
 // (1), and a combine step adds the pieces in range order and writes the
 // row. Empty rows are written as zeros, so grad_lut is fully overwritten.
-template <typename T, int V, int S, bool DOTS, bool NBP>
-__global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_rows_kernel(RowsArgs a) {
-    constexpr int NT = rows_threads(DOTS, sizeof(T));
+template <typename T, int V, int S, bool DOTS, bool NBP, int NT>
+__global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
     constexpr int NG = NT / S;  // row groups
     constexpr int K = rows_batch(V);
     constexpr int P = S * V;  // columns of the chunk
@@ -652,9 +658,7 @@ __global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_ro
     // a slot offset's low bits below the item offset: nb (NBP, P * 4 >= R) or r
     constexpr uint32_t kLow = NBP ? static_cast<uint32_t>(P * 4 - 1) : 7u;
     static_assert(!NBP || DOTS, "nb in the slot offsets serves the STE dots");
-    // DOTS: the table's LUT chunk [R][P] in LDS, f32, or f16 for an f16 LUT
-    // (the 512-thread workgroups of rows_threads)
-    using LT = std::conditional_t<NT == kRowsThreads, float, _Float16>;
+    using LT = T;  // DOTS: the table's LUT chunk [R][P] in LDS
     // the neighbour row's LDS address from one byte permute: the LUT chunk at
     // LDS offset 0 with 256-byte rows, nb (< 256) in the slot offset's low
     // byte, the lane's column offset (< 256) in the address's low byte
@@ -667,8 +671,10 @@ __global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_ro
     // unit = chunk * T + table, each XCD taking one contiguous block of units:
     // an XCD walks its chunks one at a time over every table, so the chunk's
     // slice of G is read into its L2 once
+    // (a table's parts adjacent)
     const int unit = xcd_block_unit(blockIdx.x, gridDim.x);
-    const int chunk = unit / a.tables, t = unit - chunk * a.tables;
+    const int ct = unit / a.parts, part_i = unit - ct * a.parts;
+    const int chunk = ct / a.tables, t = ct - chunk * a.tables;
     const int R = a.rows, O = a.out_f;
     const int tid = threadIdx.x, g = tid / S, j = tid % S;
     const int col = chunk * P + j * V;
@@ -710,9 +716,10 @@ __global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_ro
     }
     __syncthreads();
 
-    const int nb_all = rs[R] / K;
-    const int lo = nb_all / NG, extra = nb_all - lo * NG;
-    const int b_begin = g * lo + min(g, extra), b_end = b_begin + lo + (g < extra ? 1 : 0);
+    // the batches are dealt to the row groups of all the table's parts
+    const int nb_all = rs[R] / K, g0 = part_i * NG, gg_all = NG * a.parts;
+    const int lo = nb_all / gg_all, extra = nb_all - lo * gg_all;
+    const int b_begin = (g0 + g) * lo + min(g0 + g, extra), b_end = b_begin + lo + (g0 + g < extra ? 1 : 0);
     int cur = -1;  // row being summed
     float acc[V];
     float lkv[V];  // DOTS: L[cur] over this lane's columns
@@ -874,9 +881,13 @@ __global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_ro
     if (cur >= 0) finish(cur);
     __syncthreads();
 
-    // combine: group g writes rows g, g + groups, ...: an empty row as zeros,
-    // a row split over ranges as its pieces in range order (slot 1 of its
-    // first range, slot 0 of the others); rows inside one range are written
+    // combine: group g takes rows g, g + groups, ...: an empty row is written
+    // as zeros (by the first part), a row split over ranges of this part as its
+    // pieces in range order (slot 1 of its first range, slot 0 of the others);
+    // rows inside one range are written. Of a row that goes on in another part
+    // this part's pieces are summed and left, unscaled, in its part sums: slot 0
+    // for a row that began before the part, slot 1 for one that begins in it
+    // (merge_part_rows adds them in part order).
     const int bl = lo + 1;
     const float inv_bl = 1.0f / static_cast<float>(bl), inv_lo = 1.0f / static_cast<float>(max(lo, 1));
     auto range_of = [&](int bt) { return bt < extra * bl ? small_div(bt, inv_bl) : extra + small_div(bt - extra * bl, inv_lo); };
@@ -884,13 +895,21 @@ __global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_ro
     for (int k = g; k < R; k += NG) {
         const int fb = rs[k] / K, nbk = rs[k + 1] / K - fb;
         vec_t<float, V> w = 0.f;
+        float *sums = nullptr;
         if (nbk > 0) {
             const int gf = range_of(fb), gla = range_of(fb + nbk - 1);
             if (gf == gla) continue;
-            w = *reinterpret_cast<const vec_t<float, V> *>(part + (gf * 2 + 1) * P + j * V);
-            for (int gg = gf + 1; gg <= gla; ++gg) w += *reinterpret_cast<const vec_t<float, V> *>(part + gg * 2 * P + j * V);
+            const int ga = max(gf, g0), gb = min(gla, g0 + NG - 1);
+            if (ga > gb) continue;  // another part's row
+            w = *reinterpret_cast<const vec_t<float, V> *>(part + ((ga - g0) * 2 + (ga == gf ? 1 : 0)) * P + j * V);
+            for (int gg = ga + 1; gg <= gb; ++gg) w += *reinterpret_cast<const vec_t<float, V> *>(part + (gg - g0) * 2 * P + j * V);
+            if (ga != gf || gb != gla) sums = a.part_sums + ((static_cast<size_t>(t) * a.chunks + chunk) * a.parts + part_i) * 2 * P + (ga == gf ? P : 0);
+        } else if (part_i != 0) {
+            continue;
         }
-        if (col_ok) {
+        if (sums != nullptr) {
+            *reinterpret_cast<vec_t<float, V> *>(sums + j * V) = w;
+        } else if (col_ok) {
             float y[V];
 #pragma unroll
             for (int e = 0; e < V; ++e) y[e] = w[e] * a.scale;
@@ -910,6 +929,45 @@ __global__ __launch_bounds__(rows_threads(DOTS, sizeof(T))) void pairwise_bwd_ro
 constexpr int kReduceThreads = 1024;
 constexpr int kReduceStageBytes = 64 * 1024;  // a table's {gu, r} records staged in LDS up to 8192 items
 
+// Workgroups after the table ones (the row kernel's parts > 1): the rows of
+// table t's LUT gradient that cross parts, their part sums in part order. At
+// most parts - 1 rows.
+__device__ __forceinline__ void merge_part_rows(const ReduceArgs &a, int t) {
+    __shared__ int crossing[kRowsMaxParts][3], count;  // {row, first part, last part}
+    const int tid = threadIdx.x;
+    const int32_t *rs = a.row_start + static_cast<size_t>(t) * (a.rows + 1);
+    if (tid == 0) count = 0;
+    __syncthreads();
+    if (tid < a.rows) {
+        const int nb_all = rs[a.rows] / a.batch, fb = rs[tid] / a.batch, lb = rs[tid + 1] / a.batch;
+        const int all = a.groups * a.parts, lo = nb_all / all, extra = nb_all - lo * all;
+        if (fb < lb) {
+            auto part_of = [&](int bt) {  // of the row group whose range holds batch bt
+                const int g = bt < extra * (lo + 1) ? bt / (lo + 1) : extra + (bt - extra * (lo + 1)) / max(lo, 1);
+                return g / a.groups;
+            };
+            const int p0 = part_of(fb), p1 = part_of(lb - 1);
+            if (p0 != p1) {
+                const int k = atomicAdd(&count, 1);  // any order: each row is summed by itself
+                crossing[k][0] = tid;
+                crossing[k][1] = p0;
+                crossing[k][2] = p1;
+            }
+        }
+    }
+    __syncthreads();
+    for (int k = 0; k < count; ++k) {
+        const int row = crossing[k][0], p0 = crossing[k][1], p1 = crossing[k][2];
+        for (int col = tid; col < a.out_f; col += blockDim.x) {
+            const int chunk = col / a.chunk_cols, cc = col - chunk * a.chunk_cols;
+            const float *ps = a.part_sums + (static_cast<size_t>(t) * a.chunks + chunk) * a.parts * 2 * a.chunk_cols + cc;
+            float sum = ps[(2 * p0 + 1) * a.chunk_cols];
+            for (int p = p0 + 1; p <= p1; ++p) sum += ps[2 * p * a.chunk_cols];
+            a.grad_lut[(static_cast<size_t>(t) * a.rows + row) * a.out_f + col] = sum * a.scale;
+        }
+    }
+}
+
 __global__ __launch_bounds__(kReduceThreads) void pairwise_bwd_reduce_kernel(ReduceArgs a) {
     constexpr int kWaves = kReduceThreads / kWave, kU = 4;
     __shared__ float tp[kWaves * 8];
@@ -917,12 +975,17 @@ __global__ __launch_bounds__(kReduceThreads) void pairwise_bwd_reduce_kernel(Red
     // and leave as whole lines after the walk, instead of as scattered
     // 8-byte stores
     extern __shared__ __align__(16) uint64_t gstage[];  // [items]
+    if (static_cast<int>(blockIdx.x) >= a.tables) {  // uniform per workgroup
+        merge_part_rows(a, blockIdx.x - a.tables);
+        return;
+    }
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint64_t *rec_t = a.rec + static_cast<size_t>(t) * a.items;
     const uint32_t *so = a.slot_off + static_cast<size_t>(t) * a.slots;
     const float *pd = a.pdot + static_cast<size_t>(t) * a.chunks * a.slots;
-    const int n_slots = a.row_start[static_cast<size_t>(t) * (a.rows + 1) + a.rows];
+    const int32_t *rs = a.row_start + static_cast<size_t>(t) * (a.rows + 1);
+    const int n_slots = rs[a.rows];
     float tv[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) tv[c] = 0.f;
@@ -1008,7 +1071,6 @@ constexpr uint32_t kPadSlot = 0x80000000u;  // sorted-entry flag of a row's padd
 constexpr int kItemRoleMaxTables = 192;
 constexpr int kItemRoleMinWgs = 32;
 constexpr int kItemChunk = 32;
-constexpr int kCus = 256;               // gfx950 (MI355X)
 constexpr int kItemRoleRowBytes = 448;
 
 struct FusedArgs {
@@ -1796,13 +1858,11 @@ hipError_t allow_lds(K kernel, int bytes) {
     return allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes);
 }
 
-template <typename T, int V, int S, bool DOTS>
-hipError_t launch_rows_vs(const RowsArgs &args, const BackwardPlan &p, int tables, hipStream_t stream) {
-    auto kernel = DOTS && p.rows_nb_pack ? pairwise_bwd_rows_kernel<T, V, S, DOTS, DOTS>
-                                         : pairwise_bwd_rows_kernel<T, V, S, DOTS, false>;
+template <typename T, int V, int S, bool DOTS, int NT>
+hipError_t launch_rows_nt(const RowsArgs &args, const BackwardPlan &p, int tables, hipStream_t stream) {
+    auto kernel = DOTS && p.rows_nb_pack ? pairwise_bwd_rows_kernel<T, V, S, DOTS, DOTS, NT>
+                                         : pairwise_bwd_rows_kernel<T, V, S, DOTS, false, NT>;
     const int lds = DOTS ? p.rows_lds_dots_bytes : p.rows_lds_bytes;
-    constexpr int threads = rows_threads(DOTS, sizeof(T));
-    if (threads != (DOTS ? p.rows_dots_threads : kRowsThreads)) return hipErrorInvalidConfiguration;  // plan mismatch
     if constexpr (rows_nb_perm(DOTS, sizeof(T), S, V)) {
         // the byte-permute neighbour reads address the LUT chunk from LDS
         // address 0: the kernel must have no static LDS (the dynamic array
@@ -1818,8 +1878,15 @@ hipError_t launch_rows_vs(const RowsArgs &args, const BackwardPlan &p, int table
         }
     }
     if (hipError_t e = allow_lds(kernel, lds); e != hipSuccess) return e;
-    return launch_kernel(TROPNN_KERNEL_BACKWARD_TABLE, kernel, dim3(tables * p.rows_chunks), dim3(threads), lds,
+    return launch_kernel(TROPNN_KERNEL_BACKWARD_TABLE, kernel, dim3(tables * p.rows_chunks * args.parts), dim3(NT), lds,
                          stream, args);
+}
+
+template <typename T, int V, int S, bool DOTS>
+hipError_t launch_rows_vs(const RowsArgs &args, const BackwardPlan &p, int tables, hipStream_t stream) {
+    if constexpr (DOTS)
+        if (p.rows_dots_threads == kRowsSmall) return launch_rows_nt<T, V, S, DOTS, kRowsSmall>(args, p, tables, stream);
+    return launch_rows_nt<T, V, S, DOTS, kRowsThreads>(args, p, tables, stream);
 }
 
 template <typename T, int V, bool DOTS>
@@ -1979,7 +2046,7 @@ hipError_t launch_scatter(const uint64_t *gurec, const int32_t *index_offsets, c
                          dim3(kScatterThreads), p.scatter_lds_bytes, stream, s);
 }
 
-BackwardPlan plan_backward(const Dims &d, int ste_mode) {
+BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
     BackwardPlan p{};
     p.full = (ste_mode & 0xff) == TROPNN_STE_FULL;
     const int esize = d.lut_dtype == TROPNN_LUT_F16 ? 2 : 4;
@@ -2001,16 +2068,29 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode) {
     // then the row groups' slot-offset rings, 16 bytes per thread
     p.rows_ring_off = p.rows_part_off + (kRowsThreads / p.rows_slices) * 2 * rows_chunk * 4;
     p.rows_lds_bytes = p.rows_ring_off + kRowsThreads * 16;
-    // with dots: the LUT chunk [R][P] f32 at offset 0 (its rows' addresses
+    // with dots: the LUT chunk [R][P] at offset 0 (its rows' addresses
     // are then byte permutes), then the row starts and the split-row slots
     p.rows_lut_off = 0;
-    // (in the LUT's element type for an f16 LUT, with rows_threads' 512-thread
-    // workgroups)
-    p.rows_dots_threads = rows_threads(true, esize);
+    // (in the LUT's element type)
     p.rows_dots_rs_off = (d.rows * rows_chunk * esize + 15) & ~15;
     p.rows_dots_part_off = (p.rows_dots_rs_off + (d.rows + 1) * 4 + 15) & ~15;
-    p.rows_dots_ring_off = p.rows_dots_part_off + (p.rows_dots_threads / p.rows_slices) * 2 * rows_chunk * 4;
-    p.rows_lds_dots_bytes = p.rows_dots_ring_off + p.rows_dots_threads * 16;
+    for (p.rows_dots_threads = kRowsSmall;; p.rows_dots_threads = kRowsThreads) {
+        p.rows_dots_ring_off = p.rows_dots_part_off + (p.rows_dots_threads / p.rows_slices) * 2 * rows_chunk * 4;
+        p.rows_lds_dots_bytes = p.rows_dots_ring_off + p.rows_dots_threads * 16;
+        if (p.rows_dots_threads == kRowsThreads || p.rows_lds_dots_bytes <= kRowsSmallLds) break;
+    }
+    // parts of a (table, chunk), where the units alone leave a quarter of the
+    // GPU's workgroup slots empty: enough for two rounds, at least four batches
+    // a row group
+    {
+        const long long units = static_cast<long long>(d.tables) * p.rows_chunks;
+        const int slots = kCus * (p.rows_dots_threads == kRowsSmall ? 2 : 1);
+        long long parts = units > 0 && units * 4 < slots * 3ll ? (2 * slots + units - 1) / units : 1;
+        const long long most = d.items / (4ll * p.rows_batch * (p.rows_dots_threads / p.rows_slices));
+        if (parts > most) parts = most;
+        if (parts > kRowsMaxParts) parts = kRowsMaxParts;
+        p.rows_parts = parts < 1 || lean ? 1 : static_cast<int>(parts);
+    }
     // the neighbour row fits below the item offset (a multiple of P * 4 bytes)
     p.rows_nb_pack = rows_chunk * 4 >= d.rows;
     p.sort_lds_bytes = ((kSortThreads / kWave) * d.rows + d.rows + kSortThreads / kWave) * 4 + (kSortThreads / kWave) * 8 * 4;
@@ -2133,6 +2213,9 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode) {
         off = align16(off + static_cast<size_t>(p.rows_chunks) * d.items * rows_chunk * sizeof(float));
         p.ws_pdot = off;
         if (!p.full) off = align16(off + static_cast<size_t>(d.tables) * p.rows_chunks * p.sort_slots * sizeof(float));
+        p.ws_part_sums = off;
+        if (!p.full && p.rows_parts > 1)
+            off = align16(off + static_cast<size_t>(d.tables) * p.rows_chunks * p.rows_parts * 2 * rows_chunk * sizeof(float));
         p.workspace_bytes = off;
     }
     return p;
@@ -2311,6 +2394,8 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     r.items = d.items;
     r.chunks = p.rows_chunks;
     r.lut_off = p.rows_lut_off;
+    r.parts = dots ? p.rows_parts : 1;
+    r.part_sums = reinterpret_cast<float *>(ws + p.ws_part_sums);
     if (hipError_t e = launch_rows(r, p, d.tables, d.lut_dtype, dots, stream); e != hipSuccess || !dots) return e;
     ReduceArgs ra{};
     ra.pdot = r.pdot;
@@ -2327,8 +2412,17 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     ra.items = d.items;
     ra.chunks = p.rows_chunks;
     ra.comps = d.comps;
+    ra.tables = d.tables;
+    ra.parts = grad_lut != nullptr ? r.parts : 1;
+    ra.part_sums = r.part_sums;
+    ra.grad_lut = grad_lut;
+    ra.groups = p.rows_dots_threads / p.rows_slices;
+    ra.batch = p.rows_batch;
+    ra.out_f = d.out_f;
+    ra.chunk_cols = p.rows_chunk;
     ra.stage = ra.gurec != nullptr && d.items <= kReduceStageBytes / 8;
-    if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_REDUCE, pairwise_bwd_reduce_kernel, dim3(d.tables),
+    if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_REDUCE, pairwise_bwd_reduce_kernel,
+                                     dim3(ra.parts > 1 ? 2 * d.tables : d.tables),
                                      dim3(kReduceThreads), ra.stage ? d.items * 8 : 0, stream, ra);
         e != hipSuccess || grad_x == nullptr)
         return e;

@@ -81,12 +81,13 @@ struct BackwardPlan {
     int rows_lut_off;   // with partial STE dots: LDS byte offset of the LUT chunk (0)
     int rows_dots_rs_off, rows_dots_part_off, rows_dots_ring_off;  // with partial STE dots: row starts, split-row slots, rings
     int rows_lds_dots_bytes;
-    int rows_dots_threads;  // threads of the row kernel's workgroup with dots (512 for an f16 LUT, else 1024)
+    int rows_dots_threads;  // threads of the row kernel's workgroup with dots (512 where two fit a CU, else 1024)
+    int rows_parts;         // with dots: workgroups that share a (table, chunk)'s batches
     bool rows_nb_pack;       // slot offsets carry the neighbour row (min-margin dots, P * 4 >= R)
     // sort kernel
     int sort_lds_bytes;
     int sort_slots;     // sorted-slot capacity of a table (items + padding to whole batches)
-    size_t ws_slot_off, ws_row_start, ws_batch_row, ws_g_chunked, ws_pdot;  // workspace byte offsets (general path)
+    size_t ws_slot_off, ws_row_start, ws_batch_row, ws_g_chunked, ws_pdot, ws_part_sums;  // workspace byte offsets (general path)
     // item kernel
     int item_vec;       // N: LUT / grad elements per lane load (16 bytes at most)
     int item_o_tiles;   // 64 * N column tiles per row
@@ -136,7 +137,9 @@ constexpr int item_wave_tables(int esize, int vec) {
 
 // ste_mode: TROPNN_STE_MIN_MARGIN or TROPNN_STE_FULL (general path only),
 // optionally with one TROPNN_BWD_INPUT_GRAD_* flag (fused path's item role).
-BackwardPlan plan_backward(const Dims &d, int ste_mode);
+// lean: the plan of the smallest workspace (no parts of a (table, chunk)), for
+// callers whose workspace is fixed.
+BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean);
 
 // Launch shape of the staged forward (gather.hip): a route kernel writes code
 // words to the caller's workspace, then a gather kernel sums the rows.
