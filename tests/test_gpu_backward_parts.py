@@ -35,6 +35,35 @@ def test_rows_split_over_parts(i, o, t, c, b, thr_std, lut_dtype):
     assert_train_parity(ref, hip, *train_step(ref, hip, x, g), tol=F16_TOL if lut_dtype == "f16" else F32_TOL, elem_rtol=1e-3)
 
 
+@pytest.mark.parametrize(
+    "i,o,t,c,b,thr_std,lut_dtype",
+    [
+        (128, 128, 136, 6, 2100, 0.3, "f32"),  # three tiles a table: workgroups of one and two tables
+        (64, 256, 3, 5, 4100, 4.0, "f32"),     # fewer units than CUs: every unit a workgroup, skewed codes
+        (32, 32, 300, 4, 3073, 0.3, "f16"),    # more tables than CUs: several whole tables a workgroup
+        (40, 26, 140, 3, 2048, 0.3, "f32"),    # two columns per lane; whole tiles
+        (32, 64, 3000, 4, 2050, 0.3, "f32"),   # gu slots past the four-item scatter kernel: a merge of its own
+        (20, 64, 7, 8, 5000, 0.3, "f32"),      # 256 rows
+    ],
+)
+def test_fused_split_over_tiles(i, o, t, c, b, thr_std, lut_dtype):
+    """The fused backward of several tiles whose (table, tile) units are dealt
+    to the workgroups: tables shared by workgroups merged, others written."""
+    ref, hip = make_pair(i, o, t, c, seed=5, thr_std=thr_std, lut_dtype=lut_dtype)
+    if lut_dtype == "f16":
+        with torch.no_grad():
+            ref.lut.copy_(ref.lut.half().float())  # the values the kernels read
+    x, g = seeded((b, i), seed=1), seeded((b, 1, o), seed=2)
+    # (element-wise bar: rows of many items, as above)
+    pair = train_step(ref, hip, x, g)
+    assert_train_parity(ref, hip, *pair, elem_rtol=1e-3)
+    first = [p.grad.clone() for p in (hip.thresholds, hip.lut)]
+    # parameter gradients alone (the merge kernel), the same sums
+    hip.zero_grad(set_to_none=True)
+    hip(x.to(DEV)).backward(g.to(DEV))
+    assert torch.equal(hip.thresholds.grad, first[0]) and torch.equal(hip.lut.grad, first[1])
+
+
 def test_allocation_free_backward_keeps_its_range():
     """A shape whose split plan needs more than the allocation-free entry
     point's 32 MiB, but whose plain one fits: still served."""

@@ -1072,6 +1072,16 @@ constexpr int kItemRoleMaxTables = 192;
 constexpr int kItemRoleMinWgs = 32;
 constexpr int kItemChunk = 32;
 constexpr int kItemRoleRowBytes = 448;
+// Split launches: from kSplitMinItems items, for rows of more than
+// kSplitRowBytes (narrower ones keep the item role, which needs no
+// workspace). Backwards measured, before and after: 136 tables x 64 rows x 128
+// f32 columns: 2048 items 29.2 -> 28.2 us, 8192 95 -> 72 us, 65536 700 -> 450
+// us; 64 columns, 8192 items 77 -> 55 us; 64 tables x 32 rows x 256 columns,
+// 2048 items 32.6 -> 23.0 us, 8192 118 -> 46 us; x 32 columns, 1100 items 13.4
+// -> 15.9 us (hence the line), 8192 items 59 -> 32 us; 300 tables x 16 rows x
+// 128 columns, 8192 items 183 -> 127 us.
+constexpr int kSplitMinItems = 2048;
+constexpr int kSplitRowBytes = 48;
 
 struct FusedArgs {
     const float *grad_out;
@@ -1096,7 +1106,63 @@ struct FusedArgs {
     float *grad_x;  // or null (no item role)
     int in_f, item_n, item_nc;
     int ir_rec_off, ir_g_off, ir_gud_off, ir_idx_off;  // LDS bytes
+    // split launches: the table_wgs workgroups share the T * tiles units
+    int tiles;
+    float *part_lut, *part_thr;  // [2 * table_wgs][R * O] and [2 * table_wgs][8]
 };
+
+// Split launches of the fused kernel (several tiles): unit u is tile u % tiles
+// of table u / tiles; workgroup w of n takes units [first(w), first(w + 1)),
+// which differ by at most one in number. A table lying in one workgroup is
+// finished there; of any other, each workgroup leaves its sums, unscaled, in
+// slot 2 w (the table it starts with) or 2 w + 1 (the one it ends with).
+__device__ __forceinline__ int split_first(int w, int n, int units) {
+    return static_cast<int>(static_cast<int64_t>(w) * units / n);
+}
+__device__ __forceinline__ int split_owner(int u, int n, int units) {  // the workgroup of unit u
+    return static_cast<int>((static_cast<int64_t>(u + 1) * n - 1) / units);
+}
+
+struct MergeArgs {
+    const float *part_lut, *part_thr;
+    float *grad_lut, *grad_thr;  // or null
+    float scale;
+    int tables, tiles, wgs, row_floats, comps;  // row_floats: R * O, a multiple of 4
+    int pieces;                                 // workgroups of a table
+};
+
+// The tables that several workgroups of a split launch share: their sums in
+// workgroup order, scaled. Block t * pieces + piece, four floats a thread.
+__device__ __forceinline__ void merge_split(const MergeArgs &m, int block) {
+    using f32x4 = vec_t<float, 4>;
+    const int t = block / m.pieces, piece = block - t * m.pieces, units = m.tables * m.tiles;
+    const int w0 = split_owner(t * m.tiles, m.wgs, units), w1 = split_owner((t + 1) * m.tiles - 1, m.wgs, units);
+    if (w0 == w1) return;  // finished in the fused kernel
+    auto slot = [&](int w) { return 2 * w + (split_first(w, m.wgs, units) / m.tiles == t ? 0 : 1); };
+    const int k = (piece * static_cast<int>(blockDim.x) + threadIdx.x) * 4;
+    if (m.grad_lut != nullptr && k < m.row_floats) {
+        f32x4 sum = *reinterpret_cast<const f32x4 *>(m.part_lut + static_cast<size_t>(slot(w0)) * m.row_floats + k);
+        constexpr int kU = 4;  // slots in flight
+        for (int w = w0 + 1; w <= w1; w += kU) {
+            f32x4 v[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                v[u] = w + u <= w1 ? *reinterpret_cast<const f32x4 *>(m.part_lut + static_cast<size_t>(slot(w + u)) * m.row_floats + k)
+                                   : f32x4(0.f);
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (w + u <= w1) sum += v[u];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] *= m.scale;
+        __builtin_nontemporal_store(sum, reinterpret_cast<f32x4 *>(m.grad_lut + static_cast<size_t>(t) * m.row_floats + k));
+    }
+    if (m.grad_thr != nullptr && piece == 0 && static_cast<int>(threadIdx.x) < m.comps) {
+        float sum = m.part_thr[slot(w0) * 8 + threadIdx.x];
+        for (int w = w0 + 1; w <= w1; ++w) sum += m.part_thr[slot(w) * 8 + threadIdx.x];
+        m.grad_thr[t * m.comps + threadIdx.x] = sum;
+    }
+}
 
 constexpr int kScatterThreads = 256;  // threads of a scatter-kernel workgroup (one item)
 
@@ -1251,7 +1317,10 @@ __device__ __forceinline__ void fused_item_role(const FusedArgs &a, unsigned cha
 // gu (the surrogate's division once per item, not once per lane of a row
 // group), stores {gu, r} for the scatter kernel and reduces the threshold
 // gradient.
-template <typename T, int V, int S>
+// SPLIT (several tiles, no item role): the table workgroups share the (table,
+// tile) units evenly, so that a launch of few or very many tables fills the
+// GPU; each runs through the tables its units belong to.
+template <typename T, int V, int S, bool SPLIT>
 __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(FusedArgs a) {
     constexpr int kWaves = kFusedThreads / kWave;
     constexpr int NG = kFusedThreads / S;  // row groups
@@ -1273,20 +1342,40 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
     float *part = reinterpret_cast<float *>(lds + a.part_off);             // [groups][2][pitch] split rows
     int *brow = reinterpret_cast<int *>(lds + a.brow_off);                 // [slots / K] row of each batch
 
-    if (static_cast<int>(blockIdx.x) >= a.table_wgs) {  // item role (uniform per workgroup)
-        fused_item_role<T, V, S>(a, lds);
-        return;
+    if constexpr (!SPLIT) {
+        if (static_cast<int>(blockIdx.x) >= a.table_wgs) {  // item role (uniform per workgroup)
+            fused_item_role<T, V, S>(a, lds);
+            return;
+        }
     }
-    const int t = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int R = a.rows, C = a.comps, O = a.out_f;
-    const bool single = a.items <= kFusedThreads;
+    const bool single = !SPLIT && a.items <= kFusedThreads;
     const bool need_gu = a.grad_thr != nullptr || a.gurec != nullptr;
-    const uint64_t *rec_t = a.rec + static_cast<size_t>(t) * a.items;
     const __amdgpu_buffer_rsrc_t g_rsrc = buffer_rsrc(a.grad_out, a.g_bytes);
     const __amdgpu_buffer_rsrc_t lut_rsrc = buffer_rsrc(a.lut, a.lut_bytes);
+
+    int unit = 0, unit_end = 1;
+    if constexpr (SPLIT) {
+        unit = split_first(blockIdx.x, a.table_wgs, a.tables * a.tiles);
+        unit_end = split_first(blockIdx.x + 1, a.table_wgs, a.tables * a.tiles);
+    }
+    const int unit_first = unit;
+    do {
+    // (per-lane values of a segment come from an opaque copy of the thread id:
+    // hoisted out of the segments they would stay live across them)
+    int tid = threadIdx.x;
+    if constexpr (SPLIT) __asm__ volatile("" : "+v"(tid));
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the segment: items [item0, item1) of table t
+    int t = blockIdx.x, item0 = 0, item1 = a.items;
+    if constexpr (SPLIT) {
+        t = unit / a.tiles;
+        const int tile = unit - t * a.tiles, n = min(a.tiles - tile, unit_end - unit);
+        item0 = tile * kFusedThreads;
+        item1 = min(a.items, item0 + n * kFusedThreads);
+    }
+    const uint64_t *rec_t = a.rec + static_cast<size_t>(t) * a.items;
 
     // 1. one ballot per code bit gives each item the mask of equal codes in
     //    its wave: its rank is the count below it, and the first item of
@@ -1313,7 +1402,7 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
     //    of G per XCD (workgroups are dealt to the 8 XCDs in turn, so the
     //    grad rows the walk gathers are L2 hits by then); the first ballots
     //    need the record only, and the LUT rows go to LDS after them
-    uint64_t r0 = tid < a.items ? rec_t[tid] : 0ull;
+    uint64_t r0 = item0 + tid < item1 ? rec_t[item0 + tid] : 0ull;
     float lv[kStage][CH];
     const int quads = R * O / CH;  // CH-element chunks
     {
@@ -1324,9 +1413,9 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
             buffer_row<T, CH>(lut_rsrc, q < quads ? static_cast<uint32_t>(q) * CH * sizeof(T) : kOutOfRange, tbase, lv[i]);
         }
     }
-    const uint32_t touch = static_cast<uint32_t>(t >> 3) * a.g_slice + tid * 128u;
+    const uint32_t touch = static_cast<uint32_t>(blockIdx.x >> 3) * a.g_slice + tid * 128u;
     const uint32_t pf = tid * 128u < a.g_slice ? __builtin_amdgcn_raw_buffer_load_b32(g_rsrc, touch, 0, 0) : 0u;
-    int rank = ballots(r0, min(kFusedThreads, a.items));
+    int rank = ballots(r0, min(kFusedThreads, item1 - item0));
 #pragma unroll
     for (int i = 0; i < kStage; ++i) {
         const int q = tid + i * kFusedThreads;
@@ -1351,8 +1440,8 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
     }
     __syncthreads();
 
-    for (int tile0 = 0;;) {
-        const int n_tile = min(kFusedThreads, a.items - tile0);
+    for (int tile0 = item0;;) {
+        const int n_tile = min(kFusedThreads, item1 - tile0);
         // per-lane values inside the loop come from an opaque copy of the
         // thread id: hoisted out of the loop (the scan's 32 LDS addresses,
         // the walk's lane offsets) they would stay live across the walk
@@ -1423,7 +1512,7 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
         }
         __syncthreads();
         // the G touch's only use: a word of its own after the scan carries
-        if (tile0 == 0 && tid == 0) wtot[kWaves] = static_cast<int>(pf);
+        if (tile0 == item0 && tid == 0) wtot[kWaves] = static_cast<int>(pf);
 
         // 4. walk. The batches (rows in order, K slots each) are dealt out as
         //    contiguous ranges of lo or lo + 1 batches, the longer ones to the
@@ -1513,7 +1602,7 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
         }
         if (cur >= 0) finish(cur);
         const int next = tile0 + kFusedThreads;
-        if (next < a.items) r0 = next + tid < a.items ? rec_t[next + tid] : 0ull;
+        if (next < item1) r0 = next + tid < item1 ? rec_t[next + tid] : 0ull;
         __syncthreads();
         // 5. combine: group g finishes rows g, g + groups, ...: an empty row is
         //    zero; a row split over ranges sums its pieces in range order
@@ -1587,24 +1676,29 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
                 }
             }
         }
-        if (next >= a.items) break;
+        if (next >= item1) break;
         tile0 = next;
-        rank = ballots(r0, min(kFusedThreads, a.items - tile0));
+        rank = ballots(r0, min(kFusedThreads, item1 - tile0));
         __syncthreads();
     }
 
     // 7. several tiles: the row buffer (its last rows came from the combine
-    //    step of the last tile), scaled, written once
+    //    step of the last tile), scaled, written once; of a table shared with
+    //    other workgroups, unscaled to this one's slot
+    const bool whole = !SPLIT || (item0 == 0 && item1 == a.items);
+    const int slot = 2 * blockIdx.x + (unit == unit_first ? 0 : 1);
     if (!single && a.grad_lut != nullptr) {
         __syncthreads();
+        float *dst = whole ? a.grad_lut + static_cast<size_t>(t) * R * O : a.part_lut + static_cast<size_t>(slot) * R * O;
+        const float scale = whole ? a.scale : 1.0f;
         constexpr int qp = P / CH;
-        for (int unit = tid; unit < R * qp; unit += kFusedThreads) {
-            const int k = unit / qp, c0 = (unit % qp) * CH;
+        for (int q = tid; q < R * qp; q += kFusedThreads) {
+            const int k = q / qp, c0 = (q % qp) * CH;
             if (c0 < O) {
                 float y[CH];
 #pragma unroll
-                for (int e = 0; e < CH; ++e) y[e] = rowbuf[k * P + c0 + e] * a.scale;
-                store_f32_nt<CH>(a.grad_lut + (static_cast<size_t>(t) * R + k) * O + c0, y);
+                for (int e = 0; e < CH; ++e) y[e] = rowbuf[k * P + c0 + e] * scale;
+                store_f32_nt<CH>(dst + static_cast<size_t>(k) * O + c0, y);
             }
         }
     }
@@ -1614,10 +1708,22 @@ __global__ __launch_bounds__(kFusedThreads) void pairwise_bwd_fused_kernel(Fused
         if (tid < C) {
             float sum = tp[tid];
             for (int w = 1; w < kWaves; ++w) sum += tp[w * 8 + tid];
-            a.grad_thr[t * C + tid] = sum;
+            if (whole)
+                a.grad_thr[t * C + tid] = sum;
+            else
+                a.part_thr[slot * 8 + tid] = sum;
         }
     }
+    if constexpr (SPLIT) {
+        unit += (item1 - item0 + kFusedThreads - 1) / kFusedThreads;
+        if (unit < unit_end) __syncthreads();  // the next segment rewrites the LDS
+    }
+    } while (SPLIT && unit < unit_end);
 }
+
+// The merge on its own, when no scatter kernel follows a split launch.
+constexpr int kMergeThreads = 256;
+__global__ __launch_bounds__(kMergeThreads) void pairwise_bwd_merge_kernel(MergeArgs m) { merge_split(m, blockIdx.x); }
 
 // Input gradient of the fused path: one workgroup per item expands the item's
 // {gu, r} records (one per table) into signed slots and walks the inverse
@@ -1628,6 +1734,9 @@ struct ScatterArgs {
     const int32_t *index_entries;
     float *grad_x;
     int items, in_f, tables, comps;
+    // scatter_multi: workgroups from item_wgs on merge a split fused launch
+    int item_wgs;
+    MergeArgs merge;
 };
 
 constexpr int kScatterIndex = 8;  // index words per thread in flight
@@ -1684,7 +1793,11 @@ __global__ __launch_bounds__(1024) void pairwise_bwd_scatter_multi_kernel(Scatte
     const int C = a.comps, tid = threadIdx.x, nthr = blockDim.x;
     f32x4 *gud = reinterpret_cast<f32x4 *>(lds);                      // [T * C] x 4 items
     int *idx_s = reinterpret_cast<int *>(gud + a.tables * C);          // [in_f + 1 + 2 T C + kEntries]
-    const int b0 = xcd_block_unit(blockIdx.x, gridDim.x) * kScatterItems;  // records of adjacent items share lines
+    if (static_cast<int>(blockIdx.x) >= a.item_wgs) {  // uniform per workgroup
+        merge_split(a.merge, blockIdx.x - a.item_wgs);
+        return;
+    }
+    const int b0 = xcd_block_unit(blockIdx.x, a.item_wgs) * kScatterItems;  // records of adjacent items share lines
     const int n = min(kScatterItems, a.items - b0);
     const int n_ent = 2 * a.tables * C;
     for (int t = tid; t < a.tables; t += nthr) {
@@ -1929,7 +2042,7 @@ hipError_t launch_item_typed(const ItemArgs &args, const BackwardPlan &p, hipStr
 
 template <typename T, int V, int S>
 hipError_t launch_fused_vs(const FusedArgs &args, int wgs, const BackwardPlan &p, hipStream_t stream) {
-    auto kernel = pairwise_bwd_fused_kernel<T, V, S>;
+    auto kernel = p.f_split ? pairwise_bwd_fused_kernel<T, V, S, true> : pairwise_bwd_fused_kernel<T, V, S, false>;
     if (hipError_t e = allow_lds(kernel, p.f_launch_lds); e != hipSuccess) return e;
     return launch_kernel(TROPNN_KERNEL_BACKWARD_FUSED, kernel, dim3(wgs), dim3(kFusedThreads), p.f_launch_lds,
                          stream, args);
@@ -2013,8 +2126,19 @@ hipError_t launch_scatter_wide(const uint64_t *gurec, const float *gu, const int
                          dim3(kWideThreads), 0, stream, s);
 }
 
+hipError_t launch_merge(const MergeArgs &m, hipStream_t stream) {
+    hipLaunchKernelGGL(pairwise_bwd_merge_kernel, dim3(m.tables * m.pieces), dim3(kMergeThreads), 0, stream, m);
+    return hipGetLastError();
+}
+
+// merge: a split fused launch's merge, done by this launch's last workgroups
+// (or by a launch of its own before the kernels that take one item each)
 hipError_t launch_scatter(const uint64_t *gurec, const int32_t *index_offsets, const int32_t *index_entries,
-                          float *grad_x, const Dims &d, const BackwardPlan &p, hipStream_t stream) {
+                          float *grad_x, const Dims &d, const BackwardPlan &p, const MergeArgs *merge, hipStream_t stream) {
+    const long long multi_lds = 16ll * d.tables * d.comps + 4ll * (d.in_f + 1 + 2ll * d.tables * d.comps + kEntries);
+    const bool multi = d.items >= kScatterMultiMinItems && multi_lds <= kMaxLdsBytes;
+    if (merge != nullptr && !multi)
+        if (hipError_t e = launch_merge(*merge, stream); e != hipSuccess) return e;
     if (p.wide_index) return launch_scatter_wide(gurec, nullptr, index_offsets, index_entries, grad_x, d, stream);
     ScatterArgs s{};
     s.gurec = gurec;
@@ -2031,13 +2155,18 @@ hipError_t launch_scatter(const uint64_t *gurec, const int32_t *index_offsets, c
     // 512 x 8 comparisons 116 -> 72 us; 1500 items, 300 features 6.0 -> 4.8 us.
     // Below, one item a workgroup spreads the
     // round trips wider (512 items: no difference)
-    const long long multi_lds = 16ll * d.tables * d.comps + 4 * nidx;
-    if (d.items >= kScatterMultiMinItems && multi_lds <= kMaxLdsBytes) {
+    if (multi) {
         if (hipError_t e = allow_lds(pairwise_bwd_scatter_multi_kernel, static_cast<int>(multi_lds)); e != hipSuccess) return e;
         const int threads = d.in_f <= 512 ? 256 : d.in_f <= 1024 ? 512 : 1024;
+        s.item_wgs = (d.items + kScatterItems - 1) / kScatterItems;
+        int merge_wgs = 0;
+        if (merge != nullptr) {
+            s.merge = *merge;
+            s.merge.pieces = (merge->row_floats + 4 * threads - 1) / (4 * threads);
+            merge_wgs = d.tables * s.merge.pieces;
+        }
         return launch_kernel(TROPNN_KERNEL_BACKWARD_SCATTER, pairwise_bwd_scatter_multi_kernel,
-                             dim3((d.items + kScatterItems - 1) / kScatterItems), dim3(threads),
-                             static_cast<uint32_t>(multi_lds), stream, s);
+                             dim3(s.item_wgs + merge_wgs), dim3(threads), static_cast<uint32_t>(multi_lds), stream, s);
     }
     auto kernel = nidx > kScatterIndex * kScatterThreads ? pairwise_bwd_scatter_kernel<true>
                                                          : pairwise_bwd_scatter_kernel<false>;
@@ -2182,7 +2311,14 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
         const bool by_width = (ste_mode & TROPNN_BWD_INPUT_GRAD_FUSED) != 0 ||
                               static_cast<long long>(d.tables) * d.out_f * esize <=
                                   static_cast<long long>(kItemRoleRowBytes) * (kCus - d.tables);
-        p.f_item = p.fused && d.tables <= kItemRoleMaxTables && nc >= 1 && item_bytes(1) <= kMaxLdsBytes && by_width &&
+        // split: several tiles whose (table, tile) units, dealt evenly to one
+        // workgroup per CU, take fewer tiles' time than whole tables do
+        const long long tiles = (static_cast<long long>(d.items) + kFusedThreads - 1) / kFusedThreads, units = d.tables * tiles;
+        p.f_tiles = static_cast<int>(tiles);
+        p.f_split = p.fused && !lean && d.items >= kSplitMinItems && d.out_f * esize > kSplitRowBytes &&
+                    (units + kCus - 1) / kCus < tiles * ((d.tables + kCus - 1) / kCus);
+        p.f_split_wgs = static_cast<int>(units < kCus ? units : kCus);
+        p.f_item = p.fused && !p.f_split && d.tables <= kItemRoleMaxTables && nc >= 1 && item_bytes(1) <= kMaxLdsBytes && by_width &&
                    (ste_mode & TROPNN_BWD_INPUT_GRAD_SCATTER) == 0;
         p.f_item_nc = nc;
         p.f_ir_rec_off = 0;
@@ -2201,6 +2337,11 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
     auto align16 = [](size_t v) { return (v + 15) & ~static_cast<size_t>(15); };
     if (p.fused) {
         p.workspace_bytes = p.f_item ? 0 : static_cast<size_t>(d.tables) * d.items * sizeof(uint64_t);
+        if (p.f_split) {
+            p.ws_part_lut = align16(p.workspace_bytes);
+            p.ws_part_thr = align16(p.ws_part_lut + 2ull * p.f_split_wgs * d.rows * d.out_f * sizeof(float));
+            p.workspace_bytes = p.ws_part_thr + 2ull * p.f_split_wgs * 8 * sizeof(float);
+        }
     } else {
         size_t off = align16(static_cast<size_t>(d.tables) * d.items * (p.full ? d.comps * sizeof(float) : sizeof(uint64_t)));
         p.ws_slot_off = off;
@@ -2268,7 +2409,16 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
         // table workgroups first (one per table, unless only grad_latent is
         // asked for), then the item workgroups on the CUs the table ones
         // leave free: n items each, all resident at once on MI355X
-        f.table_wgs = !item_role || grad_lut != nullptr || grad_thr != nullptr ? d.tables : 0;
+        f.table_wgs = p.f_split ? p.f_split_wgs : !item_role || grad_lut != nullptr || grad_thr != nullptr ? d.tables : 0;
+        MergeArgs m{};
+        if (p.f_split) {
+            unsigned char *ws = reinterpret_cast<unsigned char *>(workspace);
+            f.tiles = p.f_tiles;
+            f.part_lut = reinterpret_cast<float *>(ws + p.ws_part_lut);
+            f.part_thr = reinterpret_cast<float *>(ws + p.ws_part_thr);
+            m = MergeArgs{f.part_lut, f.part_thr, grad_lut, grad_thr, scale, d.tables, p.f_tiles, p.f_split_wgs,
+                          d.rows * d.out_f, d.comps, (d.rows * d.out_f + 4 * kMergeThreads - 1) / (4 * kMergeThreads)};
+        }
         int wgs = f.table_wgs;
         if (item_role) {
             int ni = device_cus(stream) - f.table_wgs;
@@ -2289,8 +2439,9 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
         }
         hipError_t e = d.lut_dtype == TROPNN_LUT_F16 ? launch_fused_typed<_Float16>(f, wgs, p, stream)
                                                       : launch_fused_typed<float>(f, wgs, p, stream);
-        if (e != hipSuccess || grad_x == nullptr || item_role) return e;
-        return launch_scatter(gurec, index_offsets, index_entries, grad_x, d, p, stream);
+        if (e != hipSuccess || item_role) return e;
+        if (grad_x == nullptr) return p.f_split ? launch_merge(m, stream) : hipSuccess;
+        return launch_scatter(gurec, index_offsets, index_entries, grad_x, d, p, p.f_split ? &m : nullptr, stream);
     }
     const bool need_gu = grad_x != nullptr || grad_thr != nullptr;
     if (p.full && need_gu) {  // full STE: per-item dots of every comparison, grad_latent
@@ -2426,7 +2577,7 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
                                      dim3(kReduceThreads), ra.stage ? d.items * 8 : 0, stream, ra);
         e != hipSuccess || grad_x == nullptr)
         return e;
-    return launch_scatter(ra.gurec, index_offsets, index_entries, grad_x, d, p, stream);
+    return launch_scatter(ra.gurec, index_offsets, index_entries, grad_x, d, p, nullptr, stream);
 }
 
 }  // namespace tropnn

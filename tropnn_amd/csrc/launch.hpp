@@ -115,6 +115,11 @@ struct BackwardPlan {
     bool f_item;
     int f_item_nc;      // items of an item-role workgroup held in LDS at once
     int f_ir_rec_off, f_ir_g_off, f_ir_gud_off, f_ir_idx_off;  // LDS bytes
+    // several tiles: the (table, tile) units shared evenly by f_split_wgs
+    // workgroups, tables that several share merged after (no item role)
+    bool f_split;
+    int f_tiles, f_split_wgs;
+    size_t ws_part_lut, ws_part_thr;
     int f_launch_lds;   // the launch's dynamic LDS: max of the two roles'
     int scatter_lds_bytes;   // gu slots [T * C] f32 + the inverse anchor index
     size_t workspace_bytes;  // fused: none with the item role, else {gu, r} [T][B] u64; general: gu, then the sort kernel's output
@@ -137,8 +142,8 @@ constexpr int item_wave_tables(int esize, int vec) {
 
 // ste_mode: TROPNN_STE_MIN_MARGIN or TROPNN_STE_FULL (general path only),
 // optionally with one TROPNN_BWD_INPUT_GRAD_* flag (fused path's item role).
-// lean: the plan of the smallest workspace (no parts of a (table, chunk)), for
-// callers whose workspace is fixed.
+// lean: the plan of the smallest workspace (no parts of a (table, chunk), no
+// split fused launch), for callers whose workspace is fixed.
 BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean);
 
 // Launch shape of the staged forward (gather.hip): a route kernel writes code
