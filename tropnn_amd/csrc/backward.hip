@@ -56,7 +56,10 @@
 //      in chunk order, gu = dot * scale * surrogate'(u), the {gu, r} record
 //      and the threshold gradient.
 //  (4) the scatter kernel above: the input gradient.
-// With the full STE (every comparison carries a dot), three launches: the
+// With the full STE (every comparison carries a dot) large batches take the
+// same four launches, the row kernel forming the C dots of every slot from the
+// row's C differences and the reduce kernel one gu per comparison
+// (plan_backward has the line). Smaller ones take three launches: the
 // full-STE item kernel (one workgroup per item, shaped like the forward: each
 // wave takes a block of tables, their current and C neighbour rows in flight,
 // one reduce-scatter completing the block's dots; gu per comparison, then the
@@ -125,6 +128,7 @@ struct SortArgs {
     uint32_t *slot_off;   // [T][slots] sorted grad-row byte offsets, kSlotPad in padding; null: no sort
     int32_t *row_start;   // [T][R + 1] first slot of each LUT row; [R] = the padded length
     int32_t *batch_row;   // [T][slots / batch] the LUT row of each batch of slots
+    int32_t *slot_of;     // [T][B] each item's slot, or null
     float *grad_thr;      // or null
     const float *grad_out;  // G [B][O]
     float *g_chunked;     // G copied chunk-major: [chunks][B][P] (P = the row kernel's chunk width)
@@ -135,6 +139,11 @@ struct SortArgs {
     int batch;                          // rows_batch(V): rows are padded to whole batches
     int copy_wgs;                       // workgroups before the table ones that copy G (0 without a sort)
 };
+
+// Full STE in the row kernel: the floats a slot's dots take in pdot, the
+// threads and items of a reduce workgroup.
+__host__ __device__ constexpr int full_pitch(int comps) { return comps <= 4 ? 4 : 8; }
+constexpr int kFullThreads = 256, kFullItems = 256;
 
 // Row kernel (general path), one workgroup per (table, column chunk).
 struct RowsArgs {
@@ -153,6 +162,7 @@ struct RowsArgs {
     float *pdot;           // [T][chunks][slots] per sorted slot: sum over the chunk's columns of G (L[nb] - L[code]), unscaled
     int items, chunks, lut_off, rs_off;  // LDS byte offsets: LUT chunk (0 with dots), row starts
     int ring_off;                        // LDS byte offset of the row groups' slot-offset rings
+    int comps;                           // full STE
     int parts;                           // workgroups that share a (table, chunk)'s batches
     float *part_sums;                    // [T][chunks][parts][2][P] sums of the rows that cross parts
 };
@@ -165,6 +175,11 @@ struct ReduceArgs {
     const uint64_t *rec;   // [T][B] route records
     uint64_t *gurec;       // [T][B] {gu bits, r} for the scatter kernel, or null
     float *grad_thr;       // or null
+    const float *margins;  // full STE: [B][T][C]
+    float *gu;             // full STE: [T][C][B], or null
+    const int32_t *slot_of;  // full STE: [T][B]
+    float *thr_part;       // full STE: [T][pieces][8], or null
+    int pieces;            // full STE: of kFullItems items
     float scale;
     int surrogate;
     int items, chunks, comps, rows, slots;
@@ -598,6 +613,7 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
                     const int code = static_cast<int>(hi[j] & 0xffffu) & (R - 1), r = static_cast<int>(hi[j] >> 16) & 7;
                     const uint32_t low = a.nb_pack ? static_cast<uint32_t>((code ^ (1 << r)) & (R - 1)) : static_cast<uint32_t>(r);
                     const int pos = cnt[wave * R + code] + rank[j];
+                    if (a.slot_of != nullptr) a.slot_of[static_cast<size_t>(t) * a.items + b] = pos;
                     so[pos] = (static_cast<uint32_t>(b) * static_cast<uint32_t>(a.chunk_cols) * 4u) | low;
                     if ((pos & (K - 1)) == 0) br[pos / K] = code;  // K is 4 or 8
                 }
@@ -649,7 +665,12 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
 // row crossing the range's start (end) leaves its sum in the group's slot 0
 // (1), and a combine step adds the pieces in range order and writes the
 // row. Empty rows are written as zeros, so grad_lut is fully overwritten.
-template <typename T, int V, int S, bool DOTS, bool NBP, int NT>
+// FULL (full STE): the dots of every comparison, against the row's C
+// differences L[code ^ 2^c] - L[code], which a row's slots share and the lanes
+// hold in registers while the row is open; one reduce-scatter per comparison
+// and batch, each lane storing its slot's dots as whole 16-byte pieces,
+// pdot[t][chunk][slot][4 or 8] (the first C count).
+template <typename T, int V, int S, bool DOTS, bool NBP, int NT, bool FULL>
 __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
     constexpr int NG = NT / S;  // row groups
     constexpr int K = rows_batch(V);
@@ -658,6 +679,7 @@ __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
     // a slot offset's low bits below the item offset: nb (NBP, P * 4 >= R) or r
     constexpr uint32_t kLow = NBP ? static_cast<uint32_t>(P * 4 - 1) : 7u;
     static_assert(!NBP || DOTS, "nb in the slot offsets serves the STE dots");
+    static_assert(!FULL || (DOTS && !NBP), "the full STE reads every neighbour row");
     using LT = T;  // DOTS: the table's LUT chunk [R][P] in LDS
     // the neighbour row's LDS address from one byte permute: the LUT chunk at
     // LDS offset 0 with 256-byte rows, nb (< 256) in the slot offset's low
@@ -725,7 +747,12 @@ __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
     float lkv[V];  // DOTS: L[cur] over this lane's columns
 #pragma unroll
     for (int e = 0; e < V; ++e) acc[e] = lkv[e] = 0.f;
-    float *pd = DOTS ? a.pdot + (static_cast<size_t>(t) * a.chunks + chunk) * a.slots : nullptr;
+    float *pd = DOTS ? a.pdot + (static_cast<size_t>(t) * a.chunks + chunk) * (FULL ? full_pitch(a.comps) : 1) * a.slots : nullptr;
+    float diff[FULL ? TROPNN_MAX_COMPARISONS : 1][V];  // FULL: L[cur ^ 2^c] - L[cur]
+#pragma unroll
+    for (int c = 0; c < (FULL ? TROPNN_MAX_COMPARISONS : 1); ++c)
+#pragma unroll
+        for (int e = 0; e < V; ++e) diff[c][e] = 0.f;
     auto finish = [&](int k) {  // row k's sum over this range
         if (gl == nullptr) return;
         const int fb = rs[k] / K, lb = rs[k + 1] / K - 1;
@@ -811,12 +838,52 @@ __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
 #pragma unroll
                 for (int e = 0; e < V; ++e) lkv[e] = static_cast<float>(lv[e]);
             }
+            if constexpr (FULL) {
+#pragma unroll
+                for (int c = 0; c < TROPNN_MAX_COMPARISONS; ++c)
+                    if (c < a.comps) {  // uniform
+                        const vec_t<LT, V> nv = *reinterpret_cast<const vec_t<LT, V> *>(lut_s + ((k ^ (1 << c)) & (R - 1)) * P + j * V);
+#pragma unroll
+                        for (int e = 0; e < V; ++e) diff[c][e] = static_cast<float>(nv[e]) - lkv[e];
+                    }
+            }
         }
 #pragma unroll
         for (int u = 0; u < K; ++u)
 #pragma unroll
             for (int e = 0; e < V; ++e) acc[e] += gv[u][e];
-        if constexpr (DOTS) {
+        if constexpr (FULL) {
+            float dots[K / KR][TROPNN_MAX_COMPARISONS];  // of the slot each lane holds
+#pragma unroll
+            for (int c = 0; c < TROPNN_MAX_COMPARISONS; ++c) {
+#pragma unroll
+                for (int h = 0; h < K / KR; ++h) dots[h][c] = 0.f;
+                if (c < a.comps) {  // uniform
+#pragma unroll
+                    for (int h = 0; h < K / KR; ++h) {
+                        float d[KR];
+#pragma unroll
+                        for (int q = 0; q < KR; ++q) {
+                            d[q] = 0.f;
+#pragma unroll
+                            for (int e = 0; e < V; ++e) d[q] += gv[h * KR + q][e] * diff[c][e];
+                        }
+                        dots[h][c] = reduce_scatter<S, KR>(d, j);
+                    }
+                }
+            }
+            const int q = (j / (S / KR)) & (KR - 1);
+            if (j % (S / KR) == 0 && live)
+#pragma unroll
+                for (int h = 0; h < K / KR; ++h) {
+                    float *to = pd + static_cast<size_t>(bt * K + h * KR + q) * full_pitch(a.comps);
+#pragma unroll
+                    for (int c = 0; c < TROPNN_MAX_COMPARISONS; c += 4)
+                        if (c < a.comps)  // uniform
+                            __builtin_nontemporal_store(vec_t<float, 4>{dots[h][c], dots[h][c + 1], dots[h][c + 2], dots[h][c + 3]},
+                                                        reinterpret_cast<vec_t<float, 4> *>(to + c));
+                }
+        } else if constexpr (DOTS) {
             // a group past its range has cur's row (or row 0) and reads zeros
             const int kk = max(cur, 0);
             // the batch's neighbour rows, all reads issued before the dots
@@ -870,13 +937,13 @@ __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
         // up its dots, then takes the next window (one wave's LDS accesses
         // complete in order)
         if (((i + 1) & (W - 1)) == 0) {
-            if constexpr (DOTS) flush(i / W);
+            if constexpr (DOTS && !FULL) flush(i / W);
             *reinterpret_cast<vec_t<uint32_t, 4> *>(ring + 4 * j) = wnext;
             wnext = window((i + 1) / W + 1);
         }
         ring_offsets((i + 1) & (W - 1), off);
     }
-    if constexpr (DOTS)
+    if constexpr (DOTS && !FULL)
         if ((i & (W - 1)) != 0) flush(i / W);  // the last, partial window
     if (cur >= 0) finish(cur);
     __syncthreads();
@@ -1049,6 +1116,107 @@ __global__ __launch_bounds__(kReduceThreads) void pairwise_bwd_reduce_kernel(Red
             a.grad_thr[t * a.comps + tid] = sum;
         }
     }
+}
+
+// The same with the full STE, item by item: gu_c = (sum over the chunks of
+// dot_c) * scale * surrogate'(m_c) with the comparison's own margin, left as
+// gu[t][c][b] for the scatter kernel. A slot's dots are one or two 16-byte
+// reads a chunk at the item's slot, gu runs along the items. Bound by the
+// scattered reads' round trips (a line per margin row and slot), so kFullItems
+// items a workgroup, many of them: one workgroup a table walking its slots took
+// 28.5 us where this takes 12.7 (136 tables, 2048 items, 128 columns; 4096
+// items of 16 tables, 1000 columns: 186 -> 13; 512 items a workgroup 5 % faster
+// at 8192 items of 136 tables, 10 % slower with 16 tables). C is a template
+// argument for the margins' vector loads. The threshold sums (-gu_c) of a
+// table's pieces add up in order in thr_merge.
+template <int C>
+__global__ __launch_bounds__(kFullThreads) void pairwise_bwd_reduce_full_kernel(ReduceArgs a) {
+    using f32x4 = vec_t<float, 4>;
+    constexpr int CP = full_pitch(C);
+    constexpr int kWaves = kFullThreads / kWave, kU = kFullItems / kFullThreads;
+    __shared__ float tp[kWaves * 8];
+    const int units = a.tables * a.pieces;
+    if (static_cast<int>(blockIdx.x) >= units) {  // uniform per workgroup
+        merge_part_rows(a, blockIdx.x - units);
+        return;
+    }
+    // adjacent tables of one piece together: an item's margins of several
+    // tables share lines
+    const int unit = xcd_block_unit(blockIdx.x, units), piece = unit / a.tables, t = unit - piece * a.tables;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int32_t *slot_of = a.slot_of + static_cast<size_t>(t) * a.items;
+    const float *pd = a.pdot + static_cast<size_t>(t) * a.chunks * CP * a.slots;
+    float tv[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) tv[c] = 0.f;
+    int b[kU], slot[kU];
+    float m[kU][C], dot[kU][CP];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+        b[u] = piece * kFullItems + u * kFullThreads + tid;
+        slot[u] = slot_of[min(b[u], a.items - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+        const float *mar = a.margins + (static_cast<size_t>(min(b[u], a.items - 1)) * a.tables + t) * C;
+#pragma unroll
+        for (int c = 0; c < C; ++c) m[u][c] = mar[c];
+#pragma unroll
+        for (int c = 0; c < CP; ++c) dot[u][c] = 0.f;
+    }
+#pragma unroll 4
+    for (int ch = 0; ch < a.chunks; ++ch)
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const float *at = pd + (static_cast<size_t>(ch) * a.slots + slot[u]) * CP;
+#pragma unroll
+            for (int h = 0; h < CP / 4; ++h) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(at + 4 * h);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dot[u][4 * h + e] += v[e];
+            }
+        }
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+            if (b[u] < a.items) {
+                const float gu = dot[u][c] * a.scale * surrogate_grad(m[u][c], a.surrogate);
+                tv[c] -= gu;
+                if (a.gu != nullptr) a.gu[(static_cast<size_t>(t) * C + c) * a.items + b[u]] = gu;
+            }
+    if (a.thr_part == nullptr) return;
+    const float sum = reduce_scatter<kWave, 8>(tv, lane);  // lane 8c: the wave's sum for comparison c
+    if ((lane & 7) == 0) tp[wave * 8 + (lane >> 3)] = sum;
+    __syncthreads();
+    if (tid < 8) {
+        float total = tp[tid];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) total += tp[w * 8 + tid];
+        a.thr_part[(static_cast<size_t>(t) * a.pieces + piece) * 8 + tid] = total;
+    }
+}
+
+// The threshold gradient from the pieces' sums, one (table, comparison) a thread.
+struct ThrMergeArgs {
+    const float *thr_part;  // [T][pieces][8], or null
+    float *grad_thr;
+    int tables, comps, pieces;
+};
+
+__device__ __forceinline__ void thr_merge(const ThrMergeArgs &a, int k) {
+    if (k >= a.tables * a.comps) return;
+    const int t = k / a.comps;
+    const float *ps = a.thr_part + static_cast<size_t>(t) * a.pieces * 8 + (k - t * a.comps);
+    float sum = 0.f;
+#pragma unroll 8
+    for (int p = 0; p < a.pieces; ++p) sum += ps[p * 8];
+    a.grad_thr[k] = sum;
+}
+
+__global__ __launch_bounds__(kFullThreads) void pairwise_bwd_thr_merge_kernel(ThrMergeArgs a) {
+    thr_merge(a, blockIdx.x * kFullThreads + threadIdx.x);
 }
 
 // ------------------------------------------------------------------ fused row kernel
@@ -1730,13 +1898,16 @@ __global__ __launch_bounds__(kMergeThreads) void pairwise_bwd_merge_kernel(Merge
 // anchor index as the item kernel does.
 struct ScatterArgs {
     const uint64_t *gurec;  // [T][B]
+    const float *gu;        // scatter_multi, full STE: [T][C][B] in place of the records
     const int32_t *index_offsets;
     const int32_t *index_entries;
     float *grad_x;
     int items, in_f, tables, comps;
-    // scatter_multi: workgroups from item_wgs on merge a split fused launch
+    // scatter_multi: workgroups from item_wgs on merge a split fused launch, or
+    // add up the full STE's threshold sums
     int item_wgs;
     MergeArgs merge;
+    ThrMergeArgs thr;
 };
 
 constexpr int kScatterIndex = 8;  // index words per thread in flight
@@ -1794,13 +1965,32 @@ __global__ __launch_bounds__(1024) void pairwise_bwd_scatter_multi_kernel(Scatte
     f32x4 *gud = reinterpret_cast<f32x4 *>(lds);                      // [T * C] x 4 items
     int *idx_s = reinterpret_cast<int *>(gud + a.tables * C);          // [in_f + 1 + 2 T C + kEntries]
     if (static_cast<int>(blockIdx.x) >= a.item_wgs) {  // uniform per workgroup
-        merge_split(a.merge, blockIdx.x - a.item_wgs);
+        if (a.thr.thr_part != nullptr)
+            thr_merge(a.thr, (blockIdx.x - a.item_wgs) * nthr + tid);
+        else
+            merge_split(a.merge, blockIdx.x - a.item_wgs);
         return;
     }
     const int b0 = xcd_block_unit(blockIdx.x, a.item_wgs) * kScatterItems;  // records of adjacent items share lines
     const int n = min(kScatterItems, a.items - b0);
     const int n_ent = 2 * a.tables * C;
-    for (int t = tid; t < a.tables; t += nthr) {
+    if (a.gu != nullptr) {  // uniform: every comparison's slot as it is
+        stage_index(idx_s, a.index_offsets, a.index_entries, a.in_f, n_ent, 0, a.in_f + 1 + n_ent + kEntries, tid, nthr);
+        const bool vec = n == kScatterItems && (a.items & 3) == 0;
+#pragma unroll 4
+        for (int k = tid; k < a.tables * C; k += nthr) {
+            const float *src = a.gu + static_cast<size_t>(k) * a.items + b0;
+            f32x4 v;
+            if (vec) {
+                v = *reinterpret_cast<const f32x4 *>(src);
+            } else {
+#pragma unroll
+                for (int i = 0; i < kScatterItems; ++i) v[i] = src[min(i, n - 1)];
+            }
+            gud[k] = v;
+        }
+    }
+    for (int t = tid; t < a.tables && a.gu == nullptr; t += nthr) {
         const uint64_t *src = a.gurec + static_cast<size_t>(t) * a.items + b0;
         uint64_t rr[kScatterItems];
 #pragma unroll
@@ -1815,7 +2005,7 @@ __global__ __launch_bounds__(1024) void pairwise_bwd_scatter_multi_kernel(Scatte
             gud[t * C + c] = v;
         }
     }
-    if (tid >= a.tables)
+    if (tid >= a.tables && a.gu == nullptr)
         stage_index(idx_s, a.index_offsets, a.index_entries, a.in_f, n_ent, 0, a.in_f + 1 + n_ent + kEntries, tid, nthr);
     __syncthreads();
     const int *off_s = idx_s, *ent_s = idx_s + a.in_f + 1;
@@ -1973,8 +2163,15 @@ hipError_t allow_lds(K kernel, int bytes) {
 
 template <typename T, int V, int S, bool DOTS, int NT>
 hipError_t launch_rows_nt(const RowsArgs &args, const BackwardPlan &p, int tables, hipStream_t stream) {
-    auto kernel = DOTS && p.rows_nb_pack ? pairwise_bwd_rows_kernel<T, V, S, DOTS, DOTS, NT>
-                                         : pairwise_bwd_rows_kernel<T, V, S, DOTS, false, NT>;
+    if constexpr (DOTS && V <= 4)  // the full STE's plan takes at most four columns per lane
+        if (p.full_rows) {
+            auto kernel = pairwise_bwd_rows_kernel<T, V, S, true, false, NT, true>;
+            if (hipError_t e = allow_lds(kernel, p.rows_lds_dots_bytes); e != hipSuccess) return e;
+            return launch_kernel(TROPNN_KERNEL_BACKWARD_TABLE, kernel, dim3(tables * p.rows_chunks * args.parts), dim3(NT),
+                                 p.rows_lds_dots_bytes, stream, args);
+        }
+    auto kernel = DOTS && p.rows_nb_pack ? pairwise_bwd_rows_kernel<T, V, S, DOTS, DOTS, NT, false>
+                                         : pairwise_bwd_rows_kernel<T, V, S, DOTS, false, NT, false>;
     const int lds = DOTS ? p.rows_lds_dots_bytes : p.rows_lds_bytes;
     if constexpr (rows_nb_perm(DOTS, sizeof(T), S, V)) {
         // the byte-permute neighbour reads address the LUT chunk from LDS
@@ -2126,6 +2323,11 @@ hipError_t launch_scatter_wide(const uint64_t *gurec, const float *gu, const int
                          dim3(kWideThreads), 0, stream, s);
 }
 
+long long scatter_multi_lds(const Dims &d) {
+    return 16ll * d.tables * d.comps + 4ll * (d.in_f + 1 + 2ll * d.tables * d.comps + kEntries);
+}
+bool scatter_multi_ok(const Dims &d) { return d.items >= kScatterMultiMinItems && scatter_multi_lds(d) <= kMaxLdsBytes; }
+
 hipError_t launch_merge(const MergeArgs &m, hipStream_t stream) {
     hipLaunchKernelGGL(pairwise_bwd_merge_kernel, dim3(m.tables * m.pieces), dim3(kMergeThreads), 0, stream, m);
     return hipGetLastError();
@@ -2133,15 +2335,18 @@ hipError_t launch_merge(const MergeArgs &m, hipStream_t stream) {
 
 // merge: a split fused launch's merge, done by this launch's last workgroups
 // (or by a launch of its own before the kernels that take one item each)
-hipError_t launch_scatter(const uint64_t *gurec, const int32_t *index_offsets, const int32_t *index_entries,
+// gu, thr: the full STE's (the four-item kernel only)
+hipError_t launch_scatter(const uint64_t *gurec, const float *gu, const ThrMergeArgs &thr, const int32_t *index_offsets, const int32_t *index_entries,
                           float *grad_x, const Dims &d, const BackwardPlan &p, const MergeArgs *merge, hipStream_t stream) {
-    const long long multi_lds = 16ll * d.tables * d.comps + 4ll * (d.in_f + 1 + 2ll * d.tables * d.comps + kEntries);
-    const bool multi = d.items >= kScatterMultiMinItems && multi_lds <= kMaxLdsBytes;
+    const long long multi_lds = scatter_multi_lds(d);
+    const bool multi = scatter_multi_ok(d);
+    if (gu != nullptr && !multi) return hipErrorInvalidConfiguration;  // plan mismatch
     if (merge != nullptr && !multi)
         if (hipError_t e = launch_merge(*merge, stream); e != hipSuccess) return e;
     if (p.wide_index) return launch_scatter_wide(gurec, nullptr, index_offsets, index_entries, grad_x, d, stream);
     ScatterArgs s{};
     s.gurec = gurec;
+    s.gu = gu;
     s.index_offsets = index_offsets;
     s.index_entries = index_entries;
     s.grad_x = grad_x;
@@ -2165,6 +2370,10 @@ hipError_t launch_scatter(const uint64_t *gurec, const int32_t *index_offsets, c
             s.merge.pieces = (merge->row_floats + 4 * threads - 1) / (4 * threads);
             merge_wgs = d.tables * s.merge.pieces;
         }
+        if (thr.thr_part != nullptr) {
+            s.thr = thr;
+            merge_wgs = (d.tables * d.comps + threads - 1) / threads;
+        }
         return launch_kernel(TROPNN_KERNEL_BACKWARD_SCATTER, pairwise_bwd_scatter_multi_kernel,
                              dim3(s.item_wgs + merge_wgs), dim3(threads), static_cast<uint32_t>(multi_lds), stream, s);
     }
@@ -2179,13 +2388,26 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
     BackwardPlan p{};
     p.full = (ste_mode & 0xff) == TROPNN_STE_FULL;
     const int esize = d.lut_dtype == TROPNN_LUT_F16 ? 2 : 4;
+    // full STE, large batches: the row kernel forms every comparison's dots, a
+    // row's C differences serving all its slots, where the item kernel reads
+    // C + 1 rows per (item, table) from L2. Backward of 136 tables x 64 rows x
+    // 128 f32 columns, item -> row kernel: 2048 items 142 -> 56 us, 65536 4850 ->
+    // 1411; 64 tables x 256 rows x 512 f16 columns, 2048 items 151 -> 90; 8
+    // tables x 64 rows x 24 columns, 2048 items 27.9 -> 27.2, 4096 44 -> 29; 40
+    // tables x 8 rows x 50 columns, 1024 items 31.1 -> 22.6. Smaller ones stay
+    // (1024 items, 64 rows x 64 columns: 32 tables 26.7 us against 29.1, 8 tables
+    // 24.1 against 28.5), as do those whose dots pass 4 GiB of workspace.
+    p.full_rows = p.full && !lean && scatter_multi_ok(d) && (d.items >= 2048 || d.tables >= 40) &&
+                  static_cast<long long>(d.tables) * ((d.out_f + 63) / 64) * full_pitch(d.comps) *
+                          (d.items + 8ll * d.rows) * static_cast<long long>(sizeof(float)) <= (4ll << 30);
     // row kernel: V columns per lane (8 for rows of 64 columns or more that
     // 8 divides, else the largest divisor of the row up to 4), S lanes per
     // row group: the smallest power of two from 4 whose S * V columns cover
     // min(O, 64); 64-column chunks keep one chunk of the grad rows within an
     // XCD's L2 while the tables of the chunk are walked. Eight columns per
-    // lane halve the per-slot addressing and reduce-scatter work per column.
-    p.rows_vec = d.out_f >= kRowsChunk && d.out_f % 8 == 0 ? 8 : 4;
+    // lane halve the per-slot addressing and reduce-scatter work per column
+    // (four with the full STE, whose C differences a lane holds).
+    p.rows_vec = d.out_f >= kRowsChunk && d.out_f % 8 == 0 && !p.full_rows ? 8 : 4;
     while (p.rows_vec > 1 && d.out_f % p.rows_vec != 0) p.rows_vec >>= 1;
     p.rows_batch = rows_batch(p.rows_vec);
     p.rows_slices = 4;
@@ -2353,10 +2575,18 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
         p.ws_g_chunked = off;
         off = align16(off + static_cast<size_t>(p.rows_chunks) * d.items * rows_chunk * sizeof(float));
         p.ws_pdot = off;
-        if (!p.full) off = align16(off + static_cast<size_t>(d.tables) * p.rows_chunks * p.sort_slots * sizeof(float));
+        const bool dots = !p.full || p.full_rows;
+        if (dots)
+            off = align16(off + static_cast<size_t>(d.tables) * p.rows_chunks * p.sort_slots * (p.full ? full_pitch(d.comps) : 1) * sizeof(float));
         p.ws_part_sums = off;
-        if (!p.full && p.rows_parts > 1)
+        if (dots && p.rows_parts > 1)
             off = align16(off + static_cast<size_t>(d.tables) * p.rows_chunks * p.rows_parts * 2 * rows_chunk * sizeof(float));
+        if (p.full_rows) {
+            p.ws_slot_of = off;
+            off = align16(off + static_cast<size_t>(d.tables) * d.items * 4);
+            p.ws_thr_part = off;
+            off = align16(off + static_cast<size_t>(d.tables) * ((d.items + kFullItems - 1) / kFullItems) * 8 * sizeof(float));
+        }
         p.workspace_bytes = off;
     }
     return p;
@@ -2441,10 +2671,10 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
                                                       : launch_fused_typed<float>(f, wgs, p, stream);
         if (e != hipSuccess || item_role) return e;
         if (grad_x == nullptr) return p.f_split ? launch_merge(m, stream) : hipSuccess;
-        return launch_scatter(gurec, index_offsets, index_entries, grad_x, d, p, p.f_split ? &m : nullptr, stream);
+        return launch_scatter(gurec, nullptr, {}, index_offsets, index_entries, grad_x, d, p, p.f_split ? &m : nullptr, stream);
     }
     const bool need_gu = grad_x != nullptr || grad_thr != nullptr;
-    if (p.full && need_gu) {  // full STE: per-item dots of every comparison, grad_latent
+    if (p.full && need_gu && !p.full_rows) {  // full STE: per-item dots of every comparison, grad_latent
         ItemArgs a{};
         a.grad_out = grad_out;
         a.lut = lut;
@@ -2493,16 +2723,19 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     }
     // min-margin: the row kernel forms the STE dots, so it runs whenever any
     // gradient is asked for; the full STE needs it for the LUT gradient only
-    const bool dots = !p.full && need_gu;
+    // (the full STE past the item kernel forms them there too)
+    const bool dots = (!p.full || p.full_rows) && need_gu;
     if (grad_lut == nullptr && !dots && !(p.full && grad_thr != nullptr)) return hipSuccess;
     unsigned char *ws = reinterpret_cast<unsigned char *>(workspace);
     SortArgs so{};
     so.rec = rec64;
-    so.gu = p.full ? workspace : nullptr;
+    const bool item_gu = p.full && !p.full_rows;  // the item kernel left every gu in the workspace
+    so.gu = item_gu ? workspace : nullptr;
+    so.slot_of = dots && p.full ? reinterpret_cast<int32_t *>(ws + p.ws_slot_of) : nullptr;
     so.slot_off = grad_lut != nullptr || dots ? reinterpret_cast<uint32_t *>(ws + p.ws_slot_off) : nullptr;
     so.row_start = reinterpret_cast<int32_t *>(ws + p.ws_row_start);
     so.batch_row = reinterpret_cast<int32_t *>(ws + p.ws_batch_row);
-    so.grad_thr = p.full ? grad_thr : nullptr;
+    so.grad_thr = item_gu ? grad_thr : nullptr;
     so.grad_out = grad_out;
     so.g_chunked = reinterpret_cast<float *>(ws + p.ws_g_chunked);
     so.chunk_cols = p.rows_chunk;
@@ -2510,7 +2743,7 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     so.chunks = p.rows_chunks;
     so.batch = p.rows_batch;
     so.full = p.full ? 1 : 0;
-    so.nb_pack = dots && p.rows_nb_pack ? 1 : 0;
+    so.nb_pack = dots && p.rows_nb_pack && !p.full ? 1 : 0;
     so.items = d.items;
     so.out_f = d.out_f;
     so.comps = d.comps;
@@ -2545,6 +2778,7 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     r.items = d.items;
     r.chunks = p.rows_chunks;
     r.lut_off = p.rows_lut_off;
+    r.comps = d.comps;
     r.parts = dots ? p.rows_parts : 1;
     r.part_sums = reinterpret_cast<float *>(ws + p.ws_part_sums);
     if (hipError_t e = launch_rows(r, p, d.tables, d.lut_dtype, dots, stream); e != hipSuccess || !dots) return e;
@@ -2556,7 +2790,9 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     ra.slots = p.sort_slots;
     ra.item_shift = __builtin_ctz(static_cast<unsigned>(p.rows_chunk) * 4u);
     ra.rec = rec64;
-    ra.gurec = grad_x != nullptr ? reinterpret_cast<uint64_t *>(workspace) : nullptr;
+    ra.gurec = grad_x != nullptr && !p.full ? reinterpret_cast<uint64_t *>(workspace) : nullptr;
+    ra.gu = grad_x != nullptr && p.full ? workspace : nullptr;
+    ra.margins = margins;
     ra.grad_thr = grad_thr;
     ra.scale = scale;
     ra.surrogate = surrogate;
@@ -2571,13 +2807,39 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     ra.batch = p.rows_batch;
     ra.out_f = d.out_f;
     ra.chunk_cols = p.rows_chunk;
+    if (p.full) {
+        ra.slot_of = so.slot_of;
+        ra.pieces = (d.items + kFullItems - 1) / kFullItems;
+        ThrMergeArgs thr{};
+        thr.grad_thr = grad_thr;
+        thr.tables = d.tables;
+        thr.comps = d.comps;
+        thr.pieces = ra.pieces;
+        if (grad_thr != nullptr) thr.thr_part = ra.thr_part = reinterpret_cast<float *>(ws + p.ws_thr_part);
+        constexpr void (*kernels[])(ReduceArgs) = {
+            pairwise_bwd_reduce_full_kernel<1>, pairwise_bwd_reduce_full_kernel<2>, pairwise_bwd_reduce_full_kernel<3>,
+            pairwise_bwd_reduce_full_kernel<4>, pairwise_bwd_reduce_full_kernel<5>, pairwise_bwd_reduce_full_kernel<6>,
+            pairwise_bwd_reduce_full_kernel<7>, pairwise_bwd_reduce_full_kernel<8>};
+        static_assert(sizeof(kernels) / sizeof(kernels[0]) == TROPNN_MAX_COMPARISONS, "one per comparison count");
+        const auto kernel = kernels[d.comps - 1];
+        const int wgs = d.tables * ra.pieces + (ra.parts > 1 && grad_lut != nullptr ? d.tables : 0);
+        if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_REDUCE, kernel, dim3(wgs), dim3(kFullThreads), 0, stream, ra);
+            e != hipSuccess)
+            return e;
+        if (grad_x != nullptr)
+            return launch_scatter(nullptr, ra.gu, thr, index_offsets, index_entries, grad_x, d, p, nullptr, stream);
+        if (grad_thr == nullptr) return hipSuccess;
+        hipLaunchKernelGGL(pairwise_bwd_thr_merge_kernel, dim3((d.tables * d.comps + kFullThreads - 1) / kFullThreads),
+                           dim3(kFullThreads), 0, stream, thr);
+        return hipGetLastError();
+    }
     ra.stage = ra.gurec != nullptr && d.items <= kReduceStageBytes / 8;
     if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_REDUCE, pairwise_bwd_reduce_kernel,
                                      dim3(ra.parts > 1 ? 2 * d.tables : d.tables),
                                      dim3(kReduceThreads), ra.stage ? d.items * 8 : 0, stream, ra);
         e != hipSuccess || grad_x == nullptr)
         return e;
-    return launch_scatter(ra.gurec, index_offsets, index_entries, grad_x, d, p, nullptr, stream);
+    return launch_scatter(ra.gurec, nullptr, {}, index_offsets, index_entries, grad_x, d, p, nullptr, stream);
 }
 
 }  // namespace tropnn

@@ -87,7 +87,7 @@ struct BackwardPlan {
     // sort kernel
     int sort_lds_bytes;
     int sort_slots;     // sorted-slot capacity of a table (items + padding to whole batches)
-    size_t ws_slot_off, ws_row_start, ws_batch_row, ws_g_chunked, ws_pdot, ws_part_sums;  // workspace byte offsets (general path)
+    size_t ws_slot_off, ws_row_start, ws_batch_row, ws_g_chunked, ws_pdot, ws_part_sums, ws_slot_of, ws_thr_part;  // workspace byte offsets (general path)
     // item kernel
     int item_vec;       // N: LUT / grad elements per lane load (16 bytes at most)
     int item_o_tiles;   // 64 * N column tiles per row
@@ -96,7 +96,8 @@ struct BackwardPlan {
     int item_threads;
     bool wide_index;    // gu slots and index past one workgroup's LDS: the wide scatter kernel forms grad_latent
     int item_lds_bytes; // the item's gu slots [T * C] f32 + the inverse anchor index (0 with wide_index)
-    bool full;          // full STE (every comparison): item kernel variant, general path only
+    bool full;          // full STE (every comparison), general path only
+    bool full_rows;     // its dots in the row kernel (large batches), else in the item kernel
     // fused path (O a multiple of 4 up to 64, or of 8 up to 256, a table's LUT
     // rows within 64 KB as f32): one kernel per table does the LUT gradient, the
     // STE dots and the threshold gradient; a scatter kernel per item the input
