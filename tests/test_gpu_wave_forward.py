@@ -150,3 +150,28 @@ def test_wave_shapes_with_lut_or_output_off_16_bytes(lut_dtype, o, lut_off, out_
     with torch.no_grad():
         y_ref = ref.eval()(x).reshape(b, o) / ref.output_scale
     assert rel_err(aligned, y_ref) <= (F16_TOL if lut_dtype == "f16" else F32_TOL)
+
+
+@pytest.mark.parametrize(
+    "i,o,t,c,b,lut_dtype",
+    [
+        (33, 250, 100, 5, 1024, "f32"),  # 1000-byte rows, 25.6 M elements: the smallest batch
+        (33, 250, 100, 5, 2051, "f32"),
+        (20, 25, 32, 6, 8195, "f32"),    # 100 of 128 bytes, 8 items a wave
+        (20, 98, 70, 6, 4100, "f16"),    # 196 of 256 bytes, f16 rows on 4-byte boundaries
+        (20, 449, 40, 8, 2100, "f32"),   # two column tiles, 772 bytes of the second
+        (20, 200, 160, 7, 2051, "f32"),  # whole 16-byte pieces that end inside the tile
+    ],
+)
+def test_wave_forward_rows_that_fill_no_power_of_two(i, o, t, c, b, lut_dtype):
+    """Against the one-item kernel (whose waves split the tables differently)
+    and the oracle."""
+    ref, hip = make_pair(i, o, t, c, seed=o, thr_std=0.3, lut_dtype=lut_dtype)
+    x = seeded((b, i), seed=b)
+    hip.eval()
+    with torch.no_grad():
+        y = hip(x.to(DEV))
+        head = hip(x[:100].to(DEV))
+        tail = hip(x[-100:].to(DEV))
+    assert rel_err(y[:100].cpu(), head.cpu()) <= F32_TOL and rel_err(y[-100:].cpu(), tail.cpu()) <= F32_TOL
+    assert rel_err(y.cpu(), ref(x).detach()) <= (F16_TOL if lut_dtype == "f16" else F32_TOL)

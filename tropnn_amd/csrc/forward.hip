@@ -560,9 +560,13 @@ __global__ __launch_bounds__(kWaveThreads) void pairwise_forward_wave_kernel(Fwd
     const int g = lane >> lpr_log2, j = lane & ((1 << lpr_log2) - 1);
     const int item = item0 + g;
     const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(a.lut, a.lut_bytes);
-    const uint32_t lane_off =
-        (static_cast<uint32_t>(blockIdx.y) * static_cast<uint32_t>(a.wave_tile_bytes) + 16u * static_cast<uint32_t>(j)) |
-        (g < nitems ? 0u : kOutOfRange);
+    // the lane's 16 bytes of the row: the last ones of a row that no whole
+    // number of lanes covers end with the row (and repeat columns of the lane
+    // before: the same sums, stored twice), lanes past it read zeros
+    const int lane_byte = static_cast<int>(blockIdx.y) * a.wave_tile_bytes + 16 * j;
+    const bool lane_ok = g < nitems && lane_byte < a.row_bytes;
+    const int row_off = min(lane_byte, a.row_bytes - 16);
+    const uint32_t lane_off = static_cast<uint32_t>(row_off) | (lane_ok ? 0u : kOutOfRange);
     const uint8_t *cg = cw + (g < nitems ? g : 0) * a.codes_pitch;
     const int nblk = (a.tables + a.per_wave - 1) / a.per_wave;
 
@@ -629,12 +633,16 @@ __global__ __launch_bounds__(kWaveThreads) void pairwise_forward_wave_kernel(Fwd
             consume(b, w[q]);
         }
     }
-    if (g < nitems) {
-        float y[E];
+    if (lane_ok) {
+        typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // rows start at any element
+        float *dst = a.out + static_cast<size_t>(item) * a.out_f + row_off / static_cast<int>(sizeof(T));
 #pragma unroll
-        for (int e = 0; e < E; ++e) y[e] = tot[e] * a.scale;
-        const int col = blockIdx.y * (a.wave_tile_bytes / static_cast<int>(sizeof(T))) + j * E;
-        store_f32_nt<E>(a.out + static_cast<size_t>(item) * a.out_f + col, y);
+        for (int q = 0; q < E; q += 4) {
+            f32x4_any y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = tot[q + e] * a.scale;
+            __builtin_nontemporal_store(y, reinterpret_cast<f32x4_any *>(dst + q));
+        }
     }
 }
 
@@ -1063,19 +1071,34 @@ ForwardPlan plan_forward(const Dims &d, bool rows16) {
         }
     }
 
-    // wave-item kernel: large batches (>= kWaveMinItems items and >=
-    // kWaveMinWaves waves) whose row, or 1024-byte column tile of it, is 128
-    // to 1024 bytes (a power of two), tables summed in the multi-item
-    // kernel's blocks of at most 16; comparators, input rows and code lists
-    // within 64 KB of LDS; the LUT and the output 16-byte aligned
+    // wave-item kernel: large batches (>= kWaveMinWaves waves) whose row, or
+    // 1024-byte column tile of it, is 128 to 1024 bytes (a power of two, or at
+    // least three quarters of the next one in whole dwords), tables summed in
+    // the multi-item kernel's blocks of at most 16; comparators, input rows
+    // and code lists within 64 KB of LDS; the LUT and the output 16-byte
+    // aligned. Its waves walk the tables in turn, about 8 us before the first
+    // row is out, so it needs enough rows in flight; against the other kernels
+    // (100 tables of 32 rows, us):
+    //  - against the multi-item kernel always: 250 f32 columns, 2051 items 25.4
+    //    -> 16.9, 8192 62 -> 43; 128 columns 18.4 -> 12.4, 32 -> 24;
+    //  - against the one-item kernel with 8-byte loads (below kMultiMinItems)
+    //    from 25 M gathered elements: 250 columns, 1024 items 11.6 -> 10.0;
+    //    128 columns, 1500 items 9.0 against 10.0;
+    //  - against the one-item kernel with 16-byte loads from 60 M elements of a
+    //    LUT that an XCD's L2 holds, f16 40 M: 256 f32 columns, 2051 items 12.9
+    //    against 16.7, 3000 17.7 against 18.0, 8192 44 -> 42; 200 f16 columns,
+    //    2051 items 13.6 against 14.2, 4096 24 -> 16; from a larger LUT always
+    //    (300 tables of 64 rows, 256 f32 columns, 2051 items 84 -> 53).
     p.wave = false;
     {
         const int row_bytes = d.out_f * esize;
-        const int tile = row_bytes <= 1024 ? row_bytes : 1024;
-        const bool pow2 = (tile & (tile - 1)) == 0;
-        const int ipw = tile >= 128 ? kWave / (tile / 16) : 1;
-        if (rows16 && d.items >= kWaveMinItems && (d.items + ipw - 1) / ipw >= kWaveMinWaves && tile >= 128 &&
-            pow2 && row_bytes % tile == 0 && d.in_f <= 16384) {
+        const int tile = wave_tile(row_bytes);
+        const int ipw = tile > 0 ? kWave / (tile / 16) : 1;
+        const double elements = 1.0 * d.items * d.tables * d.out_f;
+        const bool vec16 = p.vec * esize == 16, in_l2 = static_cast<long long>(row_bytes) * d.tables * d.rows <= (4ll << 20);
+        const bool enough = d.items >= kWaveMinItems ? !(vec16 && in_l2) || elements >= (esize == 4 ? 60e6 : 40e6)
+                                                     : !vec16 && elements >= 25e6;
+        if (rows16 && enough && (d.items + ipw - 1) / ipw >= kWaveMinWaves && tile > 0 && d.in_f <= 16384) {
             const int w16 = (d.tables + kWaveBlock - 1) / kWaveBlock;
             const int per16 = (d.tables + w16 - 1) / w16;
             const int lpr = tile / 16;
@@ -1094,7 +1117,7 @@ ForwardPlan plan_forward(const Dims &d, bool rows16) {
                 p.wave_x_off = x_off;
                 p.wave_lpr_log2 = ilog2(lpr);
                 p.wave_tile_bytes = tile;
-                p.wave_tiles = row_bytes / tile;
+                p.wave_tiles = (row_bytes + tile - 1) / tile;
                 p.wave_blocks = (d.items + kWaveWaves * ipw - 1) / (kWaveWaves * ipw);
                 p.wave_lds_bytes = off;
                 p.lds_bytes = off;

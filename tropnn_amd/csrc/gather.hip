@@ -621,10 +621,14 @@ GatherPlan plan_gather(const Dims &d) {
     // Estimated microseconds of the forward.hip kernels: gathered row elements
     // over the rates they measured, 4.2 G/us for f32 rows and 4.8 for f16; where
     // the wave-item kernel reads f16 rows 7.8, and from a LUT that an XCD's L2
-    // holds 9.5 (f32 rows: 6.5)
+    // holds 9.5 (f32 rows: 6.5); its rows that fill no power of two, f32 3.4 and
+    // 4.8, f16 6 and 6.5 (1000 f16 columns, 300 tables of 64 rows, 2049 items 97 us
+    // against 113 staged; 250 f32 columns, 100 tables of 32 rows, 8192 items 43
+    // against 37; 800 columns, 136 tables of 64 rows, 2048 items 66 against 43)
     const double elements = 1e-3 * d.items * d.tables * d.out_f;  // thousands
     const bool wave_rows = row_bytes >= 128 && (row_bytes & (row_bytes - 1)) == 0, in_l2 = lut_bytes <= (4ll << 20);
-    const double rate = !wave_rows ? (esize == 4 ? 4200. : 4800.)
+    const bool ragged = !wave_rows && wave_tile(row_bytes) > 0;
+    const double rate = ragged ? (esize == 4 ? (in_l2 ? 4800. : 3400.) : in_l2 ? 6500. : 6000.) : !wave_rows ? (esize == 4 ? 4200. : 4800.)
                                    : esize == 4 ? (in_l2 ? 6500. : 4200.) : (in_l2 ? 9500. : 7800.);
     const double plain_us = elements / rate;
     // route kernel: as many quads of items as fit 64 KB of LDS with their

@@ -25,6 +25,16 @@ struct Dims {
 // LDS of one workgroup on gfx950.
 constexpr int kMaxLdsBytes = 160 * 1024;
 
+// The wave-item forward's column tile of a LUT row, bytes (0: not its shape):
+// a power of two from 128 to 1024 of which the row, whole dwords, leaves at
+// most a quarter of the lanes idle.
+inline int wave_tile(long long row_bytes) {
+    int tile = 128;
+    while (tile < 1024 && tile < row_bytes) tile <<= 1;
+    const long long padded = (row_bytes + tile - 1) / tile * tile;
+    return row_bytes % 4 == 0 && row_bytes * 4 >= padded * 3 ? tile : 0;
+}
+
 // Launch shape of the fused route + gather + scale forward.
 struct ForwardPlan {
     int vec;             // N: LUT elements per lane load (16 bytes at most)
