@@ -14,7 +14,9 @@
 // Narrow rows (O a multiple of 4 up to 64, or of 8 up to 256, one table's LUT
 // rows within 64 KB as f32; c2 is one) with the min-margin STE take the fused
 // path, two launches:
-//  (F) fused kernel, one workgroup per table. The table's LUT rows are staged
+//  (F) fused kernel, one workgroup per table (or, with several tiles of items,
+//      an even share of all the tables' tiles per workgroup, the tables that
+//      workgroups share merged by the scatter launch). The LUT rows are staged
 //      in LDS as f32; each tile of 1024 items is counting-sorted by code (one
 //      ballot per code bit, per-wave counts written by each code's first item,
 //      a DPP scan), every row padded to whole batches of 32 / V slots whose
@@ -28,20 +30,22 @@
 //      walk one thread per slot forms gu = dot * surrogate'(u), stores it as
 //      a {gu, r} record per (table, item) and sums it per comparison into the
 //      threshold gradient.
-//  (S) scatter kernel, one workgroup per item: expands the item's records into
+//  (S) scatter kernel, one workgroup per item, or four from 1024 items on:
+//      expands the item's records into
 //      (table, comparison) slots and walks the inverse anchor index into
 //      grad_latent, as the item kernel's last phase does.
 //
 // Other shapes take the general path. With the min-margin STE, four launches:
-//  (1) sort kernel, one workgroup per table: the stable counting sort of the
+//  (1) sort kernel, one workgroup per table (and others for the copy of G): the stable counting sort of the
 //      table's items by LUT row code (C wave ballots per tile of 1024 items
 //      give each item its rank among equal codes of its wave; per-wave counts
 //      and a DPP scan give row starts), written once to the workspace as the
 //      items' grad-row offsets (with the item's min-margin comparison in the
 //      low bits) with every row padded to whole batches of 8 slots, plus each
-//      batch's row; and the table's share of a chunk-major copy of G
-//      (64-column chunks, each one contiguous block).
-//  (2) row kernel, one workgroup per (table, 64-column chunk): row groups of
+//      batch's row; and a chunk-major copy of G (64-column chunks, each one
+//      contiguous block).
+//  (2) row kernel, one workgroup per (table, 64-column chunk), several where
+//      those few leave CUs idle: row groups of
 //      S lanes (V columns each) walk balanced contiguous ranges of the sorted
 //      batches, eight grad-row loads in flight per batch (padding slots read
 //      out of range: zeros), summing each row in registers; a row inside one
