@@ -312,3 +312,14 @@ def test_forward_workspace(lib):
     assert fwd(*args) == 1 and "16-byte" in _err(lib)
     args[3] = 0
     assert fwd(*args) == 1 and "tables" in _err(lib)
+
+
+def test_full_ste_copy_past_2_gib_stays_with_the_item_kernel(lib):
+    """The row kernel's chunk-major copy of G (65 columns take two chunks of 64)
+    is addressed with 32-bit offsets: a full-STE backward whose copy passes 2
+    GiB keeps the item kernel, whose plan holds no dots of the sorted slots."""
+    ws = lib.tropnn_hip_pairwise_backward_workspace_size
+    last = (1 << 31) // (128 * 4)  # items whose copy is 2 GiB
+    rows = [ws(b, 32, 65, 8, 4, ph.LUT_F32, ph.STE_FULL) for b in (last, last + 1)]
+    dots = 8 * 2 * 4 * 4 * last  # [T][chunks][slots][4] f32
+    assert rows[0] - rows[1] > dots, rows

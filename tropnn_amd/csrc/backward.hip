@@ -2400,7 +2400,9 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
     // tables x 64 rows x 24 columns, 2048 items 27.9 -> 27.2, 4096 44 -> 29; 40
     // tables x 8 rows x 50 columns, 1024 items 31.1 -> 22.6. Smaller ones stay
     // (1024 items, 64 rows x 64 columns: 32 tables 26.7 us against 29.1, 8 tables
-    // 24.1 against 28.5), as do those whose dots pass 4 GiB of workspace.
+    // 24.1 against 28.5), as do those whose dots pass 4 GiB of workspace or whose
+    // chunk-major copy of G, which the item kernel does not read, passes the
+    // 2 GiB that the row kernel's 32-bit offsets address.
     p.full_rows = p.full && !lean && scatter_multi_ok(d) && (d.items >= 2048 || d.tables >= 40) &&
                   static_cast<long long>(d.tables) * ((d.out_f + 63) / 64) * full_pitch(d.comps) *
                           (d.items + 8ll * d.rows) * static_cast<long long>(sizeof(float)) <= (4ll << 30);
@@ -2411,14 +2413,18 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
     // XCD's L2 while the tables of the chunk are walked. Eight columns per
     // lane halve the per-slot addressing and reduce-scatter work per column
     // (four with the full STE, whose C differences a lane holds).
-    p.rows_vec = d.out_f >= kRowsChunk && d.out_f % 8 == 0 && !p.full_rows ? 8 : 4;
-    while (p.rows_vec > 1 && d.out_f % p.rows_vec != 0) p.rows_vec >>= 1;
-    p.rows_batch = rows_batch(p.rows_vec);
-    p.rows_slices = 4;
-    while (p.rows_slices < 64 && p.rows_slices * p.rows_vec < (d.out_f < kRowsChunk ? d.out_f : kRowsChunk)) p.rows_slices <<= 1;
-    const int rows_chunk = p.rows_slices * p.rows_vec;
-    p.rows_chunk = rows_chunk;
-    p.rows_chunks = (d.out_f + rows_chunk - 1) / rows_chunk;
+    for (;;) {
+        p.rows_vec = d.out_f >= kRowsChunk && d.out_f % 8 == 0 && !p.full_rows ? 8 : 4;
+        while (p.rows_vec > 1 && d.out_f % p.rows_vec != 0) p.rows_vec >>= 1;
+        p.rows_batch = rows_batch(p.rows_vec);
+        p.rows_slices = 4;
+        while (p.rows_slices < 64 && p.rows_slices * p.rows_vec < (d.out_f < kRowsChunk ? d.out_f : kRowsChunk)) p.rows_slices <<= 1;
+        p.rows_chunk = p.rows_slices * p.rows_vec;
+        p.rows_chunks = (d.out_f + p.rows_chunk - 1) / p.rows_chunk;
+        if (!p.full_rows || static_cast<long long>(p.rows_chunks) * p.rows_chunk * d.items * 4 <= (1ll << 31)) break;
+        p.full_rows = false;
+    }
+    const int rows_chunk = p.rows_chunk;
     p.rows_part_off = ((d.rows + 1) * 4 + 15) & ~15;
     // then the row groups' slot-offset rings, 16 bytes per thread
     p.rows_ring_off = p.rows_part_off + (kRowsThreads / p.rows_slices) * 2 * rows_chunk * 4;
