@@ -323,3 +323,15 @@ def test_full_ste_copy_past_2_gib_stays_with_the_item_kernel(lib):
     rows = [ws(b, 32, 65, 8, 4, ph.LUT_F32, ph.STE_FULL) for b in (last, last + 1)]
     dots = 8 * 2 * 4 * 4 * last  # [T][chunks][slots][4] f32
     assert rows[0] - rows[1] > dots, rows
+
+
+@pytest.mark.parametrize("wanted", ["grad_latent", "grad_thresholds", "grad_lut"])
+def test_min_margin_copy_past_2_gib_is_refused(lib, wanted):
+    """Every gradient of the min-margin general path goes through the
+    chunk-major copy of G, the LUT's or not."""
+    items = (1 << 31) // (128 * 4) + 1  # 65 columns: G 1.02 GiB, its copy past 2 GiB
+    outs = [1 << 20 if name == wanted else None for name in ("grad_latent", "grad_thresholds", "grad_lut")]
+    fake = 1 << 20
+    rc = lib.tropnn_hip_pairwise_backward(items, 32, 65, 2, 3, fake, fake, ph.LUT_F32, fake, None, fake, fake, 1.0,
+                                          ph.STE_MIN_MARGIN, 0, *outs, fake, 1 << 60, None)
+    assert rc == 2 and "column chunks" in _err(lib)
