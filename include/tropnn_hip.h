@@ -53,8 +53,13 @@ extern "C" {
  * multiple of 4 up to 64 or of 8 up to 256) forms grad_latent. Neither: by the
  * row width, the crossover measured on independent inputs. The choice changes
  * no result bit (both forms sum in the same order), only the time and the
- * workspace size (none with FUSED). No counterpart in the reference. */
-#define TROPNN_BWD_INPUT_GRAD_FUSED 0x100   /* in the backward's first launch, whenever the shape allows
+ * workspace: none is needed with FUSED. From 2048 items on a backward whose
+ * first launch shares the tables' items evenly over the GPU may form
+ * grad_latent after it whatever the flag: the workspace size is then not 0,
+ * and FUSED without that workspace (NULL, or fewer bytes) runs the first
+ * launch per table, its parameter gradients equal to f32 rounding. No
+ * counterpart in the reference. */
+#define TROPNN_BWD_INPUT_GRAD_FUSED 0x100   /* in the backward's first launch, where the shape allows
                                                (pays where the items' codes concentrate on few LUT rows,
                                                e.g. a layer fed by another PairwiseLinear) */
 #define TROPNN_BWD_INPUT_GRAD_SCATTER 0x200 /* in a per-item kernel after it */

@@ -64,6 +64,42 @@ def test_fused_split_over_tiles(i, o, t, c, b, thr_std, lut_dtype):
     assert torch.equal(hip.thresholds.grad, first[0]) and torch.equal(hip.lut.grad, first[1])
 
 
+@pytest.mark.parametrize(
+    "i,o,t,c,b",
+    [
+        (128, 64, 136, 6, 4096),  # its split plan asks for 13 MB
+        (40, 26, 60, 3, 2100),    # two columns per lane
+    ],
+)
+def test_fused_flag_without_workspace(i, o, t, c, b):
+    """INPUT_GRAD_FUSED needs no workspace, whatever the batch: without the one
+    that a split launch asks for, the item role runs. The input gradient is the
+    split launch's bit for bit, the parameter gradients sum in another order."""
+    lib = ph.load_library()
+    mode = ph.STE_MIN_MARGIN | ph.BWD_INPUT_GRAD_FUSED
+    need = lib.tropnn_hip_pairwise_backward_workspace_size(b, i, o, t, c, ph.LUT_F32, mode)
+    assert need > 0, "the shape must take the split launch"
+    _, hip = make_pair(i, o, t, c, seed=3, thr_std=0.3)
+    hip.input_grad = "fused"
+    x, g = seeded((b, i), seed=1).to(DEV).requires_grad_(True), seeded((b, 1, o), seed=2).to(DEV)
+    hip.train()(x).backward(g)
+    _, rec, *_ = ph._route_forward(x.detach().unsqueeze(1), hip.anchors, hip.thresholds.detach(), hip.lut.detach(),
+                                   output_scale=hip.output_scale, want_record=True, return_route=False)
+    offsets, entries = ph.anchor_index(hip.anchors, i)
+    for ws_bytes in (0, need - 1):
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=DEV)
+        out = [torch.full(s, float("nan"), device=DEV) for s in ((b, i), (t, c), (t, 1 << c, o))]
+        rc = lib.tropnn_hip_pairwise_backward(
+            b, i, o, t, c, g.data_ptr(), hip.lut.data_ptr(), ph.LUT_F32, rec.data_ptr(), None, offsets.data_ptr(),
+            entries.data_ptr(), hip.output_scale, mode, 0, *(v.data_ptr() for v in out),
+            ws.data_ptr() if ws_bytes else None, ws_bytes, torch.cuda.current_stream(DEV).cuda_stream)
+        assert rc == 0, lib.tropnn_hip_last_error()
+        assert torch.equal(out[0], x.grad)
+        for got, want in zip(out[1:], (hip.thresholds.grad, hip.lut.grad)):
+            # two orders of sums of up to 4096 f32 terms: 2 sqrt(4096) roundings of 2^-24 at most
+            assert rel_err(got.cpu(), want.cpu()) <= 2 * 4096**0.5 * 2.0**-24
+
+
 def test_allocation_free_backward_keeps_its_range():
     """A shape whose split plan needs more than the allocation-free entry
     point's 32 MiB, but whose plain one fits: still served."""

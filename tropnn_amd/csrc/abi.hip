@@ -370,7 +370,14 @@ static int backward(int64_t items, int64_t in_features, int64_t out_features, in
     if (int rc = check_ste_mode(ste_mode)) return rc;
     if (surrogate != TROPNN_SURROGATE_FAST_SIGMOID_ODD && surrogate != TROPNN_SURROGATE_IZHIKEVICH)
         return fail(TROPNN_ERR_INVALID_ARGUMENT, "surrogate must be a TROPNN_SURROGATE_* value");
-    const tropnn::BackwardPlan p = tropnn::plan_backward(d, ste_mode, lean);
+    tropnn::BackwardPlan p = tropnn::plan_backward(d, ste_mode, lean);
+    // INPUT_GRAD_FUSED needs no workspace: without one a split launch (which
+    // merges the workgroups' sums from it) gives way to the item role
+    if (p.f_split && (ste_mode & TROPNN_BWD_INPUT_GRAD_FUSED) != 0 &&
+        (workspace == nullptr || workspace_bytes < p.workspace_bytes)) {
+        const tropnn::BackwardPlan q = tropnn::plan_backward(d, ste_mode, true);
+        if (q.workspace_bytes == 0) p = q;
+    }
     if (d.items == 0) {
         // no items: the parameter gradients are zero (a fill kernel, not a
         // memset, so the call stays capturable in a HIP graph)

@@ -43,8 +43,10 @@ class PairwiseLinear(RoutedLinearBase):
                         "auto" decides by the row width, which is right for
                         inputs whose codes spread over the LUT; "fused" pays
                         where the items' codes concentrate on few rows, as in
-                        a layer fed by another PairwiseLinear. Results are
-                        bit-identical either way.
+                        a layer fed by another PairwiseLinear. Batches of
+                        2048 items and more whose first launch is split
+                        evenly over the GPU form it after that launch in
+                        every mode. Results are bit-identical either way.
     Attribute `cache_route_debug` (default True, as the reference's shell
     assumes) keeps `_last_indices` [B,S,T] int64 and `_last_margins`
     [B,S,T,C] f32 of the last call; False skips writing them; "lazy" writes
