@@ -100,6 +100,30 @@ def test_fused_flag_without_workspace(i, o, t, c, b):
             assert rel_err(got.cpu(), want.cpu()) <= 2 * 4096**0.5 * 2.0**-24
 
 
+@pytest.mark.parametrize("off", [0, 2])
+def test_split_launch_with_grad_lut_off_16_bytes(off):
+    """Two columns per lane (26 columns) need grad_lut aligned to two floats
+    only, in the merge of the workgroups' sums too."""
+    b, i, o, t, c = 2048, 40, 26, 140, 3
+    lib = ph.load_library()
+    _, hip = make_pair(i, o, t, c, seed=5, thr_std=0.3)
+    x, g = seeded((b, i), seed=1).to(DEV).requires_grad_(True), seeded((b, 1, o), seed=2).to(DEV)
+    hip.train()(x).backward(g)
+    _, rec, *_ = ph._route_forward(x.detach().unsqueeze(1), hip.anchors, hip.thresholds.detach(), hip.lut.detach(),
+                                   output_scale=hip.output_scale, want_record=True, return_route=False)
+    ws = torch.empty(lib.tropnn_hip_pairwise_backward_workspace_size(b, i, o, t, c, ph.LUT_F32, ph.STE_MIN_MARGIN),
+                     dtype=torch.uint8, device=DEV)
+    n = t * (1 << c) * o
+    buf = torch.full((off + n + 4,), 7.0, device=DEV)
+    rc = lib.tropnn_hip_pairwise_backward(
+        b, i, o, t, c, g.data_ptr(), hip.lut.data_ptr(), ph.LUT_F32, rec.data_ptr(), None, None, None,
+        hip.output_scale, ph.STE_MIN_MARGIN, 0, None, None, buf[off:].data_ptr(), ws.data_ptr(), ws.numel(),
+        torch.cuda.current_stream(DEV).cuda_stream)
+    assert rc == 0, lib.tropnn_hip_last_error()
+    assert torch.equal(buf[off : off + n].view_as(hip.lut.grad), hip.lut.grad)
+    assert bool((buf[:off] == 7).all()) and bool((buf[off + n :] == 7).all())
+
+
 def test_allocation_free_backward_keeps_its_range():
     """A shape whose split plan needs more than the allocation-free entry
     point's 32 MiB, but whose plain one fits: still served."""

@@ -1327,7 +1327,10 @@ __device__ __forceinline__ void merge_split(const MergeArgs &m, int block) {
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[e] *= m.scale;
-        __builtin_nontemporal_store(sum, reinterpret_cast<f32x4 *>(m.grad_lut + static_cast<size_t>(t) * m.row_floats + k));
+        // (the caller's grad_lut is aligned to two floats where rows are no multiple of four columns)
+        typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+        __builtin_nontemporal_store(static_cast<f32x4_any>(sum),
+                                    reinterpret_cast<f32x4_any *>(m.grad_lut + static_cast<size_t>(t) * m.row_floats + k));
     }
     if (m.grad_thr != nullptr && piece == 0 && static_cast<int>(threadIdx.x) < m.comps) {
         float sum = m.part_thr[slot(w0) * 8 + threadIdx.x];
