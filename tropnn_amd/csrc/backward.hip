@@ -544,6 +544,7 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
             for (int k = lane; k < R; k += kWave) cw[k] = 0;
 #pragma unroll
             for (int j = 0; j < kSortRounds; ++j) {
+                wave_lds_fence();
                 if (j < rounds) {  // uniform
                     const bool valid = s0 + (wave * rounds + j) * kWave + lane < a.items;
                     const int code = static_cast<int>(hi[j] & 0xffffu) & (R - 1);
@@ -553,8 +554,9 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
                         same &= ((code >> c) & 1) ? bc : ~bc;
                     }
                     const int below = __popcll(same & ((1ull << lane) - 1ull));
-                    const int prior = cw[code];  // (LDS operations of one wave complete in order)
+                    const int prior = cw[code];
                     rank[j] = prior + below;
+                    wave_lds_fence();
                     if (valid && below == 0) cw[code] = prior + __popcll(same);
                 }
             }

@@ -256,6 +256,15 @@ __device__ __forceinline__ int small_div(int x, float inv_d) {
     return static_cast<int>((static_cast<float>(x) + 0.5f) * inv_d);
 }
 
+// Orders a wave's LDS accesses across its lanes: what any lane stored before it,
+// every lane reads after it. The hardware completes one wave's LDS operations
+// in order, so this issues no instruction; it keeps the compiler from moving
+// or reusing the accesses around it.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Clamp an anchor into [0, n) so a corrupt anchor can never address memory
 // outside the staged input row; the host validates anchors before launch.
 __device__ __forceinline__ int clamp_index(int64_t a, int n) {
