@@ -35,6 +35,32 @@ def test_rows_split_over_parts(i, o, t, c, b, thr_std, lut_dtype):
     assert_train_parity(ref, hip, *train_step(ref, hip, x, g), tol=F16_TOL if lut_dtype == "f16" else F32_TOL, elem_rtol=1e-3)
 
 
+@pytest.mark.parametrize("o", [512, 250])  # eight columns per lane, two
+def test_row_sums_are_no_chain_of_single_items(o):
+    """The LUT gradient's distance from float64 against that of a plain f32 sum
+    of a row's items one after the other. A chain of n roundings errs by
+    sqrt(n / 2) of one, a chain of batches of 4 by half of that (and the batch
+    itself by little more than one): 0.5 to 0.6 of the plain sum, at most 0.8."""
+    b, i, t, c = 4096, 64, 128, 6
+    _, hip = make_pair(i, o, t, c, seed=5, thr_std=0.3)
+    x, g = seeded((b, i), seed=1).to(DEV), seeded((b, 1, o), seed=2)
+    hip.train()(x).backward(g.to(DEV))
+    rows = (g[:, 0].numpy(), g[:, 0].double().numpy())
+    err = [0.0, 0.0]
+    for k in range(4):
+        codes = hip._last_indices[:, 0, k].cpu().numpy()
+        for r in range(1 << c):
+            sel = codes == r
+            if not sel.any():
+                continue
+            chain, exact = rows[0][sel].cumsum(axis=0)[-1], rows[1][sel].sum(axis=0)  # (cumsum adds in order, in f32)
+            got = hip.lut.grad[k, r].double().cpu().numpy() / hip.output_scale
+            err[0] += ((got - exact) ** 2).sum()
+            err[1] += ((chain - exact) ** 2).sum()
+    print(f"[row sums] o={o} kernel / chain {(err[0] / err[1]) ** 0.5:.3f}", flush=True)
+    assert err[0] <= 0.8**2 * err[1]
+
+
 @pytest.mark.parametrize(
     "i,o,t,c,b,thr_std,lut_dtype",
     [

@@ -854,10 +854,19 @@ __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
                     }
             }
         }
+        // the batch's slots pairwise, then to the row's sum: a chain of
+        // additions per batch rather than per slot
 #pragma unroll
-        for (int u = 0; u < K; ++u)
+        for (int e = 0; e < V; ++e) {
+            float s[K / 2];
 #pragma unroll
-            for (int e = 0; e < V; ++e) acc[e] += gv[u][e];
+            for (int u = 0; u < K / 2; ++u) s[u] = gv[2 * u][e] + gv[2 * u + 1][e];
+#pragma unroll
+            for (int h = 1; h < K / 2; h <<= 1)
+#pragma unroll
+                for (int u = 0; u < K / 2; u += 2 * h) s[u] += s[u + h];
+            acc[e] += s[0];
+        }
         if constexpr (FULL) {
             float dots[K / KR][TROPNN_MAX_COMPARISONS];  // of the slot each lane holds
 #pragma unroll
