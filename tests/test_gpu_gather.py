@@ -116,6 +116,36 @@ def test_stream_gather_against_float64(b, i, o, t, c, dtype):
     assert torch.equal(forward(x, anchors, thr, lut, staged=True, record=False, debug=False)[0], staged[0])
 
 
+@pytest.mark.parametrize("b,o,t,c", [(4096, 512, 512, 6), (4100, 1024, 128, 7), (4096, 4096, 512, 4)])
+def test_stream_gather_is_as_close_to_float64_as_the_plain_forward(b, o, t, c):
+    """f16 LUT rows of unit size, whose f32 sums round: the staged forward's
+    two halves of four-table groups against the plain kernels' blocks of 16
+    tables (one run of all the groups would be 1.5 to 4 % further off)."""
+    anchors, thr, lut = layer_tensors(64, o, t, c, torch.float16, seed=b)
+    lut.copy_(torch.randn(lut.shape, generator=torch.Generator(DEV).manual_seed(1), device=DEV))
+    x = seeded((b, 64), seed=t).to(DEV)
+    lib = ph.load_library()
+    args = (b, 64, o, t, c, x.data_ptr(), anchors.data_ptr(), thr.data_ptr(), lut.data_ptr(), ph.LUT_F16, t**-0.5)
+    n = lib.tropnn_hip_pairwise_forward_workspace_size(b, 64, o, t, c, ph.LUT_F16)
+    assert n > 0, "the shape must take the staged forward"
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    rec = torch.empty(t, b, dtype=torch.int64, device=DEV)
+    codes = torch.empty(b, t, dtype=torch.uint8, device=DEV)
+    out = [torch.empty(b, o, device=DEV) for _ in range(2)]
+    stream = torch.cuda.current_stream(DEV).cuda_stream
+    rc = lib.tropnn_hip_pairwise_forward(*args, out[0].data_ptr(), None, None, None, codes.data_ptr(), stream)
+    assert rc == 0, lib.tropnn_hip_last_error()
+    rc = lib.tropnn_hip_pairwise_forward_ws(*args, out[1].data_ptr(), rec.data_ptr(), None, None, None, ws.data_ptr(), n, stream)
+    assert rc == 0, lib.tropnn_hip_last_error()
+    exact = torch.zeros(b, o, dtype=torch.float64, device=DEV)
+    for k in range(t):
+        exact += lut[k].double()[codes[:, k].long()]
+    exact *= float(torch.tensor(t**-0.5, dtype=torch.float32))
+    plain, staged = (float((v.double() - exact).norm() / exact.norm()) for v in out)
+    print(f"[stream gather] {b} x {o}, {t} tables: plain {plain:.4g}, staged {staged:.4g}", flush=True)
+    assert 0 < staged <= plain
+
+
 def test_non_finite_rows_stay_in_their_items():
     """An infinity or NaN of the LUT reaches exactly the items whose codes name
     its row: padding slots and absent tables read zeros, not other rows."""

@@ -388,12 +388,16 @@ struct StreamWordsArgs {
     int nblk;     // item blocks
     int gs;       // groups of four tables per stage
     int stages;
+    int half;     // stages summed before the sums are put by (0: one run of all)
+    int stagger;  // chunk pairs that do so in turn, a stage apart
 };
 
 constexpr int kStreamWThreads = 1024;
 constexpr int kStreamWChunk = 64;                       // bytes of every LUT row in a workgroup's column chunk
 constexpr int kStreamWSlots = kStreamWThreads / (kStreamWChunk / 16);  // 256 thread quads, IPT items each
 constexpr int kStreamWBufBytes = 64 * 1024;             // a stage's LUT rows, at most (two buffers)
+constexpr int kStreamWhole = 32;                        // tables summed in one run, at most
+constexpr int kStreamStagger = 8;                       // a power of two
 
 // One 16-byte LDS-direct load per lane: LDS address lds_base (wave-uniform)
 // + 16 * lane. Written in assembly so that the compiler does not know that it
@@ -430,13 +434,20 @@ __device__ __forceinline__ float add_f16_pair(uint32_t a, uint32_t b) {  // half
 // per wave read, against 10 for rows at random and 17 when all slots read the
 // same table (measured, 16-wave workgroups). A group's four rows are summed
 // as (r0 + r1) + (r2 + r3), which that reordering leaves unchanged, then added
-// to the item's sum. (f32 rows keep forward.hip's streamed gather, which sums
+// to the item's sum. More than kStreamWhole tables are summed in two halves, the
+// first half's sums lying in the output meanwhile (a second set of sums has no
+// room in the registers): one run of 128 group sums is further from float64
+// than the 16-table blocks of the wave-item kernel, two runs of 64 are closer
+// (512 tables of 0.02 N(0, 1) 3.37e-8 in one run, 3.27e-8 in blocks, 2.97e-8 in
+// halves; 128 tables of N(0, 1) 2.93e-8, 2.88e-8, 2.86e-8; 32 tables equal).
+// (f32 rows keep forward.hip's streamed gather, which sums
 // the tables one after the other as the reference does: a sum of hundreds of
 // f32 rows in another order differs from it in the last places, where f16
 // rows' sums are mostly exact.)
-//   1 GiB of f16 LUT (512 tables of 256 rows of 4096 columns): 4096 items 477 us
-// against the wave-item kernel's 1975 us; 8192 items 805 us against the 1060 us
-// of forward.hip's streamed gather. The sums alone (LDS and the mixed-precision
+//   1 GiB of f16 LUT (512 tables of 256 rows of 4096 columns): 4096 items 478 us
+// against the wave-item kernel's 1975 us; 8192 items 815 us against the 1060 us
+// of forward.hip's streamed gather (459 and 776 us in one run; the stores of the
+// first half's sums are what the halves cost). The sums alone (LDS and the mixed-precision
 // adds, which issue at half the rate of f32 ones) would take 2.2 us a stage
 // where a stage takes 3.2 to 3.7 us.
 template <int IPT>
@@ -444,6 +455,7 @@ __global__ __launch_bounds__(kStreamWThreads) void pairwise_stream_words_kernel(
     constexpr int PE = 8;  // f16 columns of a 16-byte piece
     constexpr int COLS = kStreamWChunk / 2;
     using u32x4 = vec_t<uint32_t, 4>;
+    using f32x4 = vec_t<float, 4>;
     extern __shared__ __align__(16) unsigned char lds[];  // at LDS address 0: two buffers of [gs][rows][4][64] bytes, kStreamWBufBytes apart
     const int R = a.rows;
     const int unit = xcd_block_unit(blockIdx.x, gridDim.x);
@@ -528,6 +540,18 @@ __global__ __launch_bounds__(kStreamWThreads) void pairwise_stream_words_kernel(
     issue(0, 0);
     touch(1);
     int gi = 0;
+    // the stage before which the sums are put by and the one after which they
+    // are taken back: not the same for all of an XCD's chunks, or the whole
+    // output would move at once
+    const int turn = (chunk >> 1) & (a.stagger - 1);
+    const int put = a.half != 0 ? a.half + turn : -1, get = a.half != 0 ? a.stages - 1 - turn : -1;
+    // the thread's piece of its first item's output row (formed where it is
+    // used: it would stay live across the sums)
+    auto output = [&](int cols) {
+        int t = threadIdx.x;
+        __asm__ volatile("" : "+v"(t));
+        return a.out + (static_cast<size_t>(blk) * (kStreamWSlots * IPT) + (t >> 2) * IPT) * a.out_f + chunk * COLS + (t & 3) * cols;
+    };
     for (int s = 0; s < a.stages; ++s) {
         // this stage's rows (issued a stage ago) have landed, and every wave
         // is past its reads of the other buffer
@@ -537,6 +561,18 @@ __global__ __launch_bounds__(kStreamWThreads) void pairwise_stream_words_kernel(
         asm volatile("" ::"v"(touched));
         if (s + 1 < a.stages) issue(s + 1, (s + 1) & 1);
         touch(s + 2);
+        if (s == put) {  // uniform; on the way while this stage is summed
+            float *to = output(4);  // (a store's four lanes fill 64 bytes)
+#pragma unroll
+            for (int i = 0; i < IPT; ++i, to += a.out_f) {
+                if (b0 + i < a.items)
+#pragma unroll
+                    for (int q = 0; q < PE; q += 4)
+                        *reinterpret_cast<f32x4 *>(to + 4 * q) = f32x4{acc[i][q], acc[i][q + 1], acc[i][q + 2], acc[i][q + 3]};
+#pragma unroll
+                for (int e = 0; e < PE; ++e) acc[i][e] = 0.f;
+            }
+        }
         const int g1 = min(a.gs, groups - s * a.gs);
         for (int g = 0; g < g1; ++g) {
             const uint32_t *nsrc = wsrc + static_cast<size_t>(min(++gi, groups - 1)) * a.pitch;
@@ -558,18 +594,29 @@ __global__ __launch_bounds__(kStreamWThreads) void pairwise_stream_words_kernel(
                 for (int e = 0; e < PE; ++e) acc[i][e] += p0[e] + p1[e];
             }
         }
+        if (s == get) {  // uniform
+            const float *from = output(4);
+#pragma unroll
+            for (int i = 0; i < IPT; ++i, from += a.out_f)
+                if (b0 + i < a.items)
+#pragma unroll
+                    for (int q = 0; q < PE; q += 4) {
+                        const f32x4 first = *reinterpret_cast<const f32x4 *>(from + 4 * q);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][q + e] = first[e] + acc[i][q + e];
+                    }
+        }
         off01 ^= 0x00010000u;
         off23 ^= 0x00010000u;
     }
-    const int col = chunk * COLS + piece * PE;
+    float *to = output(PE);
 #pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int b = b0 + i;
-        if (b < a.items) {
+    for (int i = 0; i < IPT; ++i, to += a.out_f) {
+        if (b0 + i < a.items) {
             float y[PE];
 #pragma unroll
             for (int e = 0; e < PE; ++e) y[e] = acc[i][e] * a.scale;
-            store_f32_nt<PE>(a.out + static_cast<size_t>(b) * a.out_f + col, y);
+            store_f32_nt<PE>(to, y);
         }
     }
 }
@@ -658,6 +705,7 @@ GatherPlan plan_gather(const Dims &d) {
         const int groups = (d.tables + 3) / 4;
         p.stream_gs = kStreamWBufBytes / (d.rows * 256);
         while (p.stream_gs > 1 && p.stream_gs / 2 >= groups) p.stream_gs /= 2;  // a power of two
+        if (d.tables > kStreamWhole && p.stream_gs >= groups) p.stream_gs /= 2;  // two halves, at a stage's end
         p.stream_stages = (groups + p.stream_gs - 1) / p.stream_gs;
         p.lds_bytes = kStreamWBufBytes + p.stream_gs * d.rows * 256;
         // items per thread: the least estimated time. A stage of 64 KB takes
@@ -781,7 +829,7 @@ hipError_t launch_gather(const Dims &d, const GatherPlan &p, const float *x, con
         return e;
     if (p.stream) {
         StreamWordsArgs s{lut, words, out, scale, d.items, d.out_f, d.tables, d.rows, p.pitch, p.stream_nblk, p.stream_gs,
-                          p.stream_stages};
+                          p.stream_stages, d.tables > kStreamWhole ? p.stream_stages / 2 : 0, p.stream_stages >= 4 * kStreamStagger ? kStreamStagger : 1};
         return launch_stream_words_ipt(s, p, stream);
     }
     SliceArgs s{};
