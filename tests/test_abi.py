@@ -303,6 +303,9 @@ def test_forward_workspace(lib):
     assert ws(8192, 128, 128, 136, 6, ph.LUT_F16) == 0  # the wave-item kernel's rows: not enough to gain
     assert ws(4096, 1024, 4096, 512, 8, ph.LUT_F16) == 32 * 16 * 4096  # stream gather
     assert ws(512, 1024, 4096, 512, 8, ph.LUT_F16) == 0  # too few items for the LUT to stream
+    assert ws(2048, 256, 512, 512, 6, ph.LUT_F16) == 0  # 71 us in one launch, 118 us staged
+    assert ws(4095, 1024, 128, 512, 8, ph.LUT_F16) == 0  # 78 us against 269 us
+    assert ws(4096, 1024, 128, 512, 8, ph.LUT_F16) > 0  # for training only (streamed: 452 us)
     assert ws(8192, 20000, 128, 136, 6, ph.LUT_F32) == 0  # input rows beyond a workgroup's LDS
     assert ws(8192, 128, 128, 136, 9, ph.LUT_F32) == 0 and "comparisons" in _err(lib)
     fwd = lib.tropnn_hip_pairwise_forward_ws

@@ -113,10 +113,32 @@ def test_stream_gather_against_float64(b, i, o, t, c, dtype):
     # eps / 2 of it, and sqrt(t) eps for rounding errors of random sign
     err = (staged[0].double() - exact).norm() / exact.norm()
     assert float(err) <= 2.0**-24 * t**0.5
-    assert torch.equal(forward(x, anchors, thr, lut, staged=True, record=False, debug=False)[0], staged[0])
+    # without a record the 512-column layer gains nothing and keeps the one-launch kernels
+    want = forward(x, anchors, thr, lut, staged=False, record=False, debug=False) if (b, o) == (4100, 512) else staged
+    assert torch.equal(forward(x, anchors, thr, lut, staged=True, record=False, debug=False)[0], want[0])
 
 
-@pytest.mark.parametrize("b,o,t,c", [(4096, 512, 512, 6), (4100, 1024, 128, 7), (4096, 4096, 512, 4)])
+@pytest.mark.parametrize("b,o,t,c,gains", [(4096, 128, 512, 8, False), (8192, 96, 700, 8, False), (8192, 1024, 128, 8, True)])
+def test_eval_takes_the_stream_gather_only_where_it_gains(b, o, t, c, gains):
+    """An eval forward of few columns keeps the one-launch kernels at every
+    batch size (a stream gather of 8 or 12 workgroups would take several times
+    as long): the workspace, sized for training, stays untouched."""
+    anchors, thr, lut = layer_tensors(64, o, t, c, torch.float16, seed=b)
+    x = seeded((b, 64), seed=t).to(DEV)
+    lib = ph.load_library()
+    n = lib.tropnn_hip_pairwise_forward_workspace_size(b, 64, o, t, c, ph.LUT_F16)
+    out, rec = torch.empty(b, o, device=DEV), torch.empty(t, b, dtype=torch.int64, device=DEV)
+    for record in (False, True):
+        ws = torch.full((n,), 255, dtype=torch.uint8, device=DEV)
+        rc = lib.tropnn_hip_pairwise_forward_ws(
+            b, 64, o, t, c, x.data_ptr(), anchors.data_ptr(), thr.data_ptr(), lut.data_ptr(), ph.LUT_F16, 0.25,
+            out.data_ptr(), rec.data_ptr() if record else None, None, None, None, ws.data_ptr(), n,
+            torch.cuda.current_stream(DEV).cuda_stream)
+        assert rc == 0, lib.tropnn_hip_last_error()
+        assert bool((ws != 255).any()) == (record or gains)
+
+
+@pytest.mark.parametrize("b,o,t,c", [(4096, 512, 512, 6), (4100, 1024, 200, 7), (4096, 4096, 512, 4)])
 def test_stream_gather_is_as_close_to_float64_as_the_plain_forward(b, o, t, c):
     """f16 LUT rows of unit size, whose f32 sums round: the staged forward's
     two halves of four-table groups against the plain kernels' blocks of 16

@@ -267,7 +267,8 @@ int tropnn_hip_pairwise_forward_ws(int64_t items, int64_t in_features, int64_t o
         const bool rows16 = !misaligned(lut, 16) && !misaligned(output, 16);
         // the stream gather moves whole 16-byte pieces; a training forward over
         // a large f32 LUT is left to the streamed kernel of forward.hip
-        if (g.ok && (g.stream ? rows16 : !(route_record && p.stream_ok))) {
+        const bool streamed = route_record != nullptr && p.stream_ok;
+        if (g.ok && (g.stream ? rows16 && (g.stream_eval || streamed) : !streamed)) {
             if (workspace_bytes < g.workspace_bytes)
                 return fail(TROPNN_ERR_INVALID_ARGUMENT, "forward workspace of %zu bytes required, got %zu",
                             g.workspace_bytes, workspace_bytes);

@@ -28,7 +28,6 @@ constexpr int kBlockTables = 16;
 constexpr int kBlockWords = kBlockTables / 4;
 constexpr int kGatherMinItems = 256;
 constexpr long long kStreamMinLut = 32ll << 20;
-constexpr int kStreamMinItems = 4096;
 constexpr int kGatherCus = 256;              // gfx950 (MI355X)
 constexpr int kSliceLds = 156 * 1024;        // a CU's LDS for staged slices
 constexpr int kRouteLds = 78 * 1024;         // a route workgroup's LDS: two workgroups per CU
@@ -396,7 +395,7 @@ constexpr int kStreamWThreads = 1024;
 constexpr int kStreamWChunk = 64;                       // bytes of every LUT row in a workgroup's column chunk
 constexpr int kStreamWSlots = kStreamWThreads / (kStreamWChunk / 16);  // 256 thread quads, IPT items each
 constexpr int kStreamWBufBytes = 64 * 1024;             // a stage's LUT rows, at most (two buffers)
-constexpr int kStreamWhole = 32;                        // tables summed in one run, at most
+constexpr int kStreamWhole = 128;                       // tables summed in one run, at most
 constexpr int kStreamStagger = 8;                       // a power of two
 
 // One 16-byte LDS-direct load per lane: LDS address lds_base (wave-uniform)
@@ -439,7 +438,7 @@ __device__ __forceinline__ float add_f16_pair(uint32_t a, uint32_t b) {  // half
 // room in the registers): one run of 128 group sums is further from float64
 // than the 16-table blocks of the wave-item kernel, two runs of 64 are closer
 // (512 tables of 0.02 N(0, 1) 3.37e-8 in one run, 3.27e-8 in blocks, 2.97e-8 in
-// halves; 128 tables of N(0, 1) 2.93e-8, 2.88e-8, 2.86e-8; 32 tables equal).
+// halves; 128 tables 2.53e-8 every way).
 // (f32 rows keep forward.hip's streamed gather, which sums
 // the tables one after the other as the reference does: a sum of hundreds of
 // f32 rows in another order differs from it in the last places, where f16
@@ -708,15 +707,18 @@ GatherPlan plan_gather(const Dims &d) {
         if (d.tables > kStreamWhole && p.stream_gs >= groups) p.stream_gs /= 2;  // two halves, at a stage's end
         p.stream_stages = (groups + p.stream_gs - 1) / p.stream_gs;
         p.lds_bytes = kStreamWBufBytes + p.stream_gs * d.rows * 256;
-        // items per thread: the least estimated time. A stage of 64 KB takes
-        // about 1.7 us and 0.25 us more per item of a thread (measured: 1 GiB
-        // of f16 LUT, 8 items per thread, 3.7 us); one workgroup per CU
+        // items per thread: the least estimated time. A stage of 64 KB of rows
+        // comes in 1.9 us, 2.2 us more where one item block has the rows to
+        // itself, and is summed in 1.6 us and 0.26 us more per group and item
+        // of a thread; one workgroup per CU, and 9 us around it (1470 shapes of
+        // LUTs of 32 MiB to 1 GiB: 80 % within 10 %)
         double best = 0;
         const int chunks = static_cast<int>(row_bytes / kStreamWChunk);
         for (int ipt = 8; ipt >= 2; ipt >>= 1) {
             const int nblk = (d.items + kStreamWSlots * ipt - 1) / (kStreamWSlots * ipt);
             const long long wgs = static_cast<long long>(nblk) * chunks;
-            const double cost = static_cast<double>((wgs + kGatherCus - 1) / kGatherCus) * p.stream_stages * (1.7 + 0.25 * ipt);
+            const double stage = std::max(1.9 + 2.2 / nblk, 1.6 + 0.26 * ipt * p.stream_gs);
+            const double cost = 9. + static_cast<double>((wgs + kGatherCus - 1) / kGatherCus) * p.stream_stages * stage;
             if (best == 0 || cost < best) {
                 best = cost;
                 p.stream_ipt = ipt;
@@ -724,8 +726,23 @@ GatherPlan plan_gather(const Dims &d) {
                 p.wgs = static_cast<int>(wgs);
             }
         }
-        // below kStreamMinItems a launch streams the whole LUT for few items
-        if (d.items < kStreamMinItems && best > elements / 4200.) return p;
+        // against the kernels that route and gather in one launch: thousands of
+        // elements per us where the wave-item kernel or the others serve the
+        // shape, by the comparisons (the fewer rows a table has, the more
+        // items in flight share them). The chosen side was more than 5 % slower
+        // in 24 of the 1470 shapes. 512 tables of 256 rows, us, plain against
+        // staged: 128 columns, 4096 items 78 | 269, 16384 items 278 | 271; 256
+        // columns 162 | 272, 630 | 298; 512 columns 239 | 216, 998 | 316; of 64
+        // rows, 512 columns, 2048 items 71 | 118, 8192 items 262 | 130
+        constexpr double kWaveRate[] = {13e3, 13e3, 13e3, 13e3, 13e3, 10.4e3, 7.1e3, 5.1e3, 3.7e3};
+        constexpr double kItemRate[] = {6e3, 6e3, 6e3, 6e3, 6e3, 4.3e3, 3.6e3, 3.4e3, 2.9e3};
+        static_assert(sizeof kWaveRate / sizeof(double) == TROPNN_MAX_COMPARISONS + 1, "one rate per comparison count");
+        const ForwardPlan f = plan_forward(d);
+        const double plain_rate = f.wave ? (f.wave_tile_bytes < 1024 && d.comps == 8 ? 3.3e3 : kWaveRate[d.comps]) : kItemRate[d.comps];
+        p.stream_eval = best <= elements / plain_rate;
+        // (training forwards that forward.hip's streamed gather would serve always
+        // gain: 0.3 to 1.07 of its time at 612 of the shapes, three above 1.03)
+        if (!p.stream_eval && !f.stream_ok) return p;
     } else {
         // Estimated: 15 us for two launches and the route, the staged rows at
         // one line per ns and CU (three times that in several stages, which

@@ -162,6 +162,7 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean);
 struct GatherPlan {
     bool ok;                 // the shape takes it (given workspace_bytes)
     bool stream;             // stream gather, else slice gather
+    bool stream_eval;        // the stream gather gains against the one-launch kernels (else for training only, against the streamed one)
     int per, groups, pitch;  // tables per summed block; code words per item; items of a row of words
     int quads, route_lds;    // route kernel: groups of four items per workgroup
     bool route_rec_stage;
