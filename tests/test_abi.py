@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import time
 from pathlib import Path
 
 import pytest
@@ -315,6 +316,35 @@ def test_forward_workspace(lib):
     assert fwd(*args) == 1 and "16-byte" in _err(lib)
     args[3] = 0
     assert fwd(*args) == 1 and "tables" in _err(lib)
+
+
+def test_forward_planning_stays_short(lib):
+    """Narrow rows over very large batches: the launch shape is searched over
+    the distinct block sizes only, and the size query does not search. A call
+    refused for its workspace's size plans in full: 16 us when every count of
+    blocks was tried, 1 to 2 us now (the least of many, so that other load on
+    the machine does not count)."""
+    dims = (524288, 64, 4, 250, 3)
+    fake = 1 << 20
+    args = [*dims, fake, fake, fake, fake, ph.LUT_F32, 1.0, fake, None, None, None, None, fake, 16, None]
+
+    def least(fn, *a):
+        best = float("inf")
+        for _ in range(300):
+            t0 = time.perf_counter()
+            fn(*a)
+            best = min(best, time.perf_counter() - t0)
+        return best
+
+    need = lib.tropnn_hip_pairwise_forward_workspace_size(*dims, ph.LUT_F32)
+    assert need > 16
+    assert lib.tropnn_hip_pairwise_forward_ws(*args) == 1 and str(need) in _err(lib)
+    base = least(lib.tropnn_hip_pairwise_forward_ws, -1, *args[1:])  # refused before any plan
+    plan = least(lib.tropnn_hip_pairwise_forward_ws, *args) - base
+    query = least(lib.tropnn_hip_pairwise_forward_workspace_size, *dims, ph.LUT_F32)
+    base = least(lib.tropnn_hip_pairwise_forward_workspace_size, -1, *dims[1:], ph.LUT_F32)
+    print(f"plan {plan * 1e6:.2f} us, query {(query - base) * 1e6:.2f} us")
+    assert plan < 6e-6 and query - base < 2e-6
 
 
 def test_full_ste_copy_past_2_gib_stays_with_the_item_kernel(lib):

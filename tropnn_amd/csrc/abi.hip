@@ -224,7 +224,7 @@ size_t tropnn_hip_pairwise_forward_workspace_size(int64_t items, int64_t in_feat
     tropnn::Dims d{};
     if (make_dims(items, in_features, out_features, tables, comparisons, lut_dtype, d) != TROPNN_OK) return 0;
     ok();
-    const tropnn::GatherPlan g = tropnn::plan_gather(d);
+    const tropnn::GatherPlan g = tropnn::plan_gather(d, true);
     return g.ok ? g.workspace_bytes : 0;
 }
 

@@ -663,7 +663,7 @@ hipError_t launch_stream_words_ipt(const StreamWordsArgs &s, const GatherPlan &p
 
 }  // namespace
 
-GatherPlan plan_gather(const Dims &d) {
+GatherPlan plan_gather(const Dims &d, bool size_only) {
     GatherPlan p{};
     const int esize = d.lut_dtype == TROPNN_LUT_F16 ? 2 : 4;
     const long long row_bytes = static_cast<long long>(d.out_f) * esize;
@@ -682,7 +682,7 @@ GatherPlan plan_gather(const Dims &d) {
     const double rate = ragged ? (esize == 4 ? (in_l2 ? 4800. : 3400.) : in_l2 ? 6500. : 6000.) : !wave_rows ? (esize == 4 ? 4200. : 4800.)
                                    : esize == 4 ? (in_l2 ? 6500. : 4200.) : (in_l2 ? 9500. : 7800.);
     const double plain_us = elements / rate;
-    // route kernel: as many quads of items as fit 64 KB of LDS with their
+    // route kernel: as many quads of items as fit 78 KB of LDS with their
     // code lists and, where they fit too, route records; at least one quad
     const int w16 = (d.tables + kBlockTables - 1) / kBlockTables;
     p.groups = w16 * kBlockWords;
@@ -696,7 +696,7 @@ GatherPlan plan_gather(const Dims &d) {
     if (rl > kMaxLdsBytes) return p;  // input rows beyond a workgroup's LDS
     p.route_lds = static_cast<int>(rl);
     p.pitch = (d.items + 15) & ~15;
-    const long long words = static_cast<long long>(p.groups) * p.pitch;
+    p.workspace_bytes = static_cast<size_t>(p.groups) * p.pitch * sizeof(uint32_t);
 
     p.stream = esize == 2 && row_bytes % kStreamWChunk == 0 && d.rows >= 4 && lut_bytes >= kStreamMinLut;
     if (p.stream) {
@@ -751,7 +751,7 @@ GatherPlan plan_gather(const Dims &d) {
         // staged: 128 f32 columns, 136 tables of 64 rows, training: 8192 items
         // 34.0 against 36.5 us, 16384 items 57 against 51 us; 512 columns, 4096
         // items 65 against 37 us; 250 columns, 100 tables of 32 rows: 2048 items
-        // 19.2 against 20.2 us, 8192 items 62 against 37 us
+        // 19.2 against 20.2 us, 8192 items 43 against 37 us
         const double rows = static_cast<double>(d.tables) * d.rows;
         const bool one_stage = rows * kSliceBytes + 2048 <= kSliceLds;
         if (15. + 1e-3 * rows * (one_stage ? 1. : 3.) + elements / (esize == 4 ? 12000. : 16000.) > plain_us) return p;
@@ -776,6 +776,10 @@ GatherPlan plan_gather(const Dims &d) {
         p.stages = (p.blocks + p.stage_blocks - 1) / p.stage_blocks;
         p.lds_bytes = lds_for(p.stage_blocks);
         if (p.lds_bytes > kMaxLdsBytes) return p;
+        if (size_only) {
+            p.ok = true;
+            return p;
+        }
         p.zero_off = p.lds_bytes - 16;
         const int per_cu = p.lds_bytes > kSliceLds / 2 ? 1 : 2;
         const int max_thr = per_cu == 1 ? 1024 : 512;
@@ -785,8 +789,11 @@ GatherPlan plan_gather(const Dims &d) {
         double best = 0;
         const int slots = kGatherCus * per_cu;
         const int max_blk = std::max(1, std::min((d.items + kWave - 1) / kWave, 4 * slots / p.slices + 1));
-        for (int nblk = 1; nblk <= max_blk; ++nblk) {
+        for (int nblk = 1; nblk <= max_blk;) {
             const int bi = ((d.items + nblk - 1) / nblk + kWave - 1) / kWave * kWave;
+            // on to the first count of blocks with fewer items each (the cost
+            // follows from bi: 524288 items of 4 columns under 200 tries of 2049)
+            nblk = bi > kWave ? (d.items + bi - kWave - 1) / (bi - kWave) : max_blk + 1;
             int thr = (bi + p.slice_ipt - 1) / p.slice_ipt;
             thr = std::min(max_thr, (thr + kWave - 1) / kWave * kWave);
             if (thr < 256) thr = 256;
@@ -803,7 +810,6 @@ GatherPlan plan_gather(const Dims &d) {
             }
         }
     }
-    p.workspace_bytes = static_cast<size_t>(words) * sizeof(uint32_t);
     p.ok = true;
     return p;
 }

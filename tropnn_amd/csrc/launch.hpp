@@ -171,7 +171,8 @@ struct GatherPlan {
     int stream_ipt, stream_nblk, stream_gs, stream_stages;
     size_t workspace_bytes;
 };
-GatherPlan plan_gather(const Dims &d);
+// size_only: ok and workspace_bytes without the search for the launch shape
+GatherPlan plan_gather(const Dims &d, bool size_only = false);
 hipError_t launch_gather(const Dims &d, const GatherPlan &p, const float *x, const int64_t *anchors, const float *thr,
                          const void *lut, float scale, float *out, tropnn_route_record *rec, int64_t *indices,
                          float *margins, uint8_t *codes, uint32_t *words, hipStream_t stream);
