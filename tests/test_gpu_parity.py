@@ -20,6 +20,7 @@ import torch
 
 from oracle import pairwise_torch as orc
 from oracle import routing_np
+from oracle.closed_form import gradients_f64
 from tropnn_amd import PairwiseLinear, pairwise_hip_forward
 
 pytestmark = pytest.mark.gpu
@@ -120,6 +121,25 @@ def assert_train_parity(ref, hip, yx_ref, yx_hip, tol=F32_TOL, x_grad=True, elem
         bad = {k: v for k, v in elem.items() if not v <= elem_rtol}
         assert not bad, f"element-wise beyond {elem_rtol}: {bad} (all: {elem})"
     return errs
+
+
+def assert_gradients_f64(hip, x, g, grad_x, *, lut_dtype="f32", block=512):
+    """The gradients of a step over long rows against float64 on the same
+    codes, at the usual element-wise bar: there the f32 oracle's own rounding
+    (sqrt(n) eps against a cancelled sum of n items) reaches several times
+    that bar. x [B, I], g [B, 1, O]; block: items expanded to [T, O] at a time."""
+    lut = hip.lut.detach().cpu()
+    if lut_dtype == "f16":
+        lut = lut.half()  # the values the kernels read
+    parts = [gradients_f64(x[k : k + block], hip.anchors.cpu(), hip.thresholds.detach().cpu(), lut, g[k : k + block, 0],
+                           min_margin=hip.use_min_margin_ste, surrogate=hip.surrogate, output_scale=hip.tables**-0.5)
+             for k in range(0, x.shape[0], block)]
+    exact = {"grad_x": torch.cat([p[0] for p in parts]), "grad_thresholds": sum(p[1] for p in parts),
+             "grad_lut": sum(p[2] for p in parts)}
+    got = {"grad_x": grad_x, "grad_thresholds": hip.thresholds.grad, "grad_lut": hip.lut.grad}
+    elem = {k: elem_err(v, exact[k]) for k, v in got.items()}
+    print(f"[float64] {elem}", flush=True)
+    assert all(v <= ELEM_RTOL for v in elem.values()), f"element-wise beyond {ELEM_RTOL}: {elem}"
 
 
 # ---------------------------------------------------------------- route codes
