@@ -130,6 +130,24 @@ def test_fused_flag_without_workspace(i, o, t, c, b):
             assert rel_err(got.cpu(), want.cpu()) <= 2 * 4096**0.5 * 2.0**-24
 
 
+@pytest.mark.parametrize(
+    "i,o,t,c,b,lut_dtype",
+    [
+        (16, 35, 2, 5, 3000, "f32"),   # one-column pieces of G over many copy workgroups
+    ],
+)
+def test_general_path_by_size(i, o, t, c, b, lut_dtype):
+    """Either side of the general path's lines between its launch shapes."""
+    ref, hip = make_pair(i, o, t, c, seed=7, thr_std=0.3, lut_dtype=lut_dtype)
+    if lut_dtype == "f16":
+        with torch.no_grad():
+            ref.lut.copy_(ref.lut.half().float())  # the values the kernels read
+    x, g = seeded((b, i), seed=1), seeded((b, 1, o), seed=2)
+    pair = train_step(ref, hip, x, g)
+    assert_train_parity(ref, hip, *pair, elem_rtol=1e-3)
+    assert_gradients_f64(hip, x, g, pair[1][1].grad, lut_dtype=lut_dtype, block=256)
+
+
 @pytest.mark.parametrize("off", [0, 2])
 def test_split_launch_with_grad_lut_off_16_bytes(off):
     """Two columns per lane (26 columns) need grad_lut aligned to two floats

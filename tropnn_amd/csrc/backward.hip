@@ -136,7 +136,6 @@ struct SortArgs {
     float *grad_thr;      // or null
     const float *grad_out;  // G [B][O]
     float *g_chunked;     // G copied chunk-major: [chunks][B][P] (P = the row kernel's chunk width)
-    int full;             // full STE: gu of every comparison
     int nb_pack;          // slot offsets' low bits: 1: the neighbour row nb = code ^ (1 << r); 0: r
     int items, out_f, comps, rows, slots;
     int chunk_cols, chunk_vec, chunks;  // P, the row kernel's V, ceil(O / P)
@@ -471,6 +470,7 @@ __device__ void wave_exclusive_scan(int *v, int n, int lane) {
 constexpr int kSortRounds = 8;
 constexpr int kSortItems = kSortRounds * kSortThreads;
 constexpr int kCopyWgs = 256;  // copy workgroups, at most
+constexpr int kCopyRound = 4;  // pieces a thread has in flight
 
 __device__ __forceinline__ void copy_chunked(const SortArgs &a, int w, int wgs) {
     // rows (chunk, item) of P columns, a contiguous range of them per
@@ -482,7 +482,7 @@ __device__ __forceinline__ void copy_chunked(const SortArgs &a, int w, int wgs) 
     const int64_t total = static_cast<int64_t>(a.chunks) * a.items;
     const int r0 = static_cast<int>(total * w / wgs), r1 = static_cast<int>(total * (w + 1) / wgs);
     const int n = (r1 - r0) << log2p;
-    constexpr int kU = 4;  // pieces in flight per thread
+    constexpr int kU = kCopyRound;
     auto each = [&](auto vec) {
         using V = decltype(vec);
         for (int k0 = threadIdx.x; k0 < n; k0 += kU * kSortThreads) {
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(kSortThreads) void pairwise_bwd_sort_kernel(SortArg
 // reading the chunk-major copy of G (an item's piece of the chunk at
 // slot offset + chunk * B * P * 4; the offset's low 3 bits carry the item's
 // min-margin comparison r). With DOTS the workgroup also stages the table's
-// LUT chunk in LDS as f32 and, from the same grad-row pieces, forms each
+// LUT chunk in LDS (in the LUT's element type) and, from the same grad-row pieces, forms each
 // item's partial STE dot over the chunk, sum G (L[code ^ 2^r] - L[code]):
 // the current row L[code] stays in registers for the row, the neighbour rows
 // come from LDS, one reduce-scatter per batch completes the batch's dots, and
@@ -2766,16 +2766,19 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
     so.chunk_vec = p.rows_vec;
     so.chunks = p.rows_chunks;
     so.batch = p.rows_batch;
-    so.full = p.full ? 1 : 0;
     so.nb_pack = dots && p.rows_nb_pack && !p.full ? 1 : 0;
     so.items = d.items;
     so.out_f = d.out_f;
     so.comps = d.comps;
     so.rows = d.rows;
     so.slots = p.sort_slots;
-    // about 64 KB of G per copy workgroup, one to each CU at most
-    const long long copy_bytes = static_cast<long long>(d.items) * d.out_f * 4;
-    so.copy_wgs = so.slot_off == nullptr ? 0 : static_cast<int>(copy_bytes / (64 * 1024) + 1 < kCopyWgs ? copy_bytes / (64 * 1024) + 1 : kCopyWgs);
+    // a round of loads per copy workgroup, one workgroup to each CU at most.
+    // Counted in a row's pieces, not bytes: those of odd rows are one column
+    // (500 items of 33 columns, 200 tables: two workgroups by bytes, of four
+    // dependent rounds each, were the kernel's tail: 7.9 us, now 5.6)
+    const long long copy_pieces = static_cast<long long>(p.rows_chunks) * d.items * (p.rows_chunk / (p.rows_vec < 4 ? p.rows_vec : 4));
+    const long long copy_wgs = copy_pieces / (kCopyRound * kSortThreads) + 1;
+    so.copy_wgs = so.slot_off == nullptr ? 0 : static_cast<int>(copy_wgs < kCopyWgs ? copy_wgs : kCopyWgs);
     if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_SORT, pairwise_bwd_sort_kernel, dim3(d.tables + so.copy_wgs),
                                      dim3(kSortThreads), p.sort_lds_bytes, stream, so);
         e != hipSuccess || so.slot_off == nullptr)
