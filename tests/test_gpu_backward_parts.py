@@ -133,6 +133,13 @@ def test_fused_flag_without_workspace(i, o, t, c, b):
 @pytest.mark.parametrize(
     "i,o,t,c,b,lut_dtype",
     [
+        (32, 90, 128, 4, 60, "f32"),   # row kernel: 256 (table, chunk)s, workgroups of 1024 threads
+        (32, 90, 129, 4, 60, "f16"),   # 258: of 512
+        (32, 33, 512, 3, 40, "f32"),   # one column per lane: 1024 threads up to 512 (table, chunk)s
+        (32, 33, 513, 3, 40, "f32"),   # 512 threads
+        (32, 33, 6, 7, 70, "f32"),     # the LUT chunk staged eight pieces at a time, 128 rows
+        (32, 65, 4, 8, 70, "f16"),     # 256 rows, two chunks
+        (32, 33, 150, 8, 1500, "f32"), # three parts: one round of workgroups
         (16, 35, 2, 5, 3000, "f32"),   # one-column pieces of G over many copy workgroups
     ],
 )

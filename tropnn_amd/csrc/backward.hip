@@ -93,9 +93,9 @@ constexpr int kRowsBatch = 8;       // sorted slots per row-kernel batch; rows a
 constexpr int rows_batch(int vec) { return vec == 8 ? 4 : kRowsBatch; }
 
 // Threads of a row-kernel workgroup: 512 with partial dots where two such
-// workgroups fit a CU's LDS, so that one's staging and combine overlap the
-// other's walk (the LUT chunk in its element type, 32 KB at 64 columns and 256
-// f16 rows), else 1024.
+// workgroups fit a CU's LDS (the LUT chunk in its element type, 32 KB at 64
+// columns and 256 f16 rows) and there are enough of them (plan_backward), so
+// that one's staging and combine overlap the other's walk, else 1024.
 constexpr int kRowsSmall = 512;
 constexpr int kRowsMaxParts = 16;
 constexpr int kCus = 256;  // gfx950 (MI355X)
@@ -701,7 +701,13 @@ __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
     // slice of G is read into its L2 once
     // (a table's parts adjacent)
     const int unit = xcd_block_unit(blockIdx.x, gridDim.x);
-    const int ct = unit / a.parts, part_i = unit - ct * a.parts;
+    // (divisions by a count that is mostly one, a chain before the first
+    // loads: a branch round them, 122.9 -> 121.5 us at 4096 workgroups, 8.8 -> 8.3
+    // at 512 without dots)
+    const bool whole = !DOTS || a.parts == 1;  // one part: no other workgroup has batches of the table's chunk
+    int ct = unit;
+    if (!whole) ct = unit / a.parts;
+    const int part_i = whole ? 0 : unit - ct * a.parts;
     const int chunk = ct / a.tables, t = ct - chunk * a.tables;
     const int R = a.rows, O = a.out_f;
     const int tid = threadIdx.x, g = tid / S, j = tid % S;
@@ -727,26 +733,40 @@ __global__ __launch_bounds__(NT) void pairwise_bwd_rows_kernel(RowsArgs a) {
     if constexpr (DOTS) {
         // the LUT chunk: R rows of P columns (pieces of V, columns past O zero)
         const __amdgpu_buffer_rsrc_t lut_rsrc = buffer_rsrc(a.lut, a.lut_bytes);
-        for (int q = tid; q < R * S; q += NT) {
-            const int row = q / S, pc = q - row * S, c0 = chunk * P + pc * V;
-            float w[V];
-            buffer_row<T, V>(lut_rsrc,
-                             c0 < O ? static_cast<uint32_t>((static_cast<size_t>(t) * R + row) * O + c0) * sizeof(T)
-                                    : kOutOfRange,
-                             0, w);
-            vec_t<LT, V> wv;
+        auto pieces = [&](int q0, auto n) {  // q0 + u * NT, u < n: all loaded, then stored
+            constexpr int U = decltype(n)::value;
+            float w[U][V];
 #pragma unroll
-            for (int e = 0; e < V; ++e) wv[e] = static_cast<LT>(w[e]);  // exact: w came from T
-            // whole-vector LDS accesses: element by element the lanes'
-            // accesses stride by V elements and collide in the banks
-            *reinterpret_cast<vec_t<LT, V> *>(lut_s + row * P + pc * V) = wv;
-        }
+            for (int u = 0; u < U; ++u) {
+                const int q = q0 + u * NT, row = q / S, c0 = chunk * P + (q - row * S) * V;
+                buffer_row<T, V>(lut_rsrc,
+                                 c0 < O ? static_cast<uint32_t>((static_cast<size_t>(t) * R + row) * O + c0) * sizeof(T)
+                                        : kOutOfRange,
+                                 0, w[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                vec_t<LT, V> wv;
+#pragma unroll
+                for (int e = 0; e < V; ++e) wv[e] = static_cast<LT>(w[u][e]);  // exact: w came from T
+                // whole-vector LDS accesses: element by element the lanes'
+                // accesses stride by V elements and collide in the banks
+                *reinterpret_cast<vec_t<LT, V> *>(lut_s + (q0 + u * NT) * V) = wv;  // (P = S * V)
+            }
+        };
+        // narrow pieces are many round trips: eight at a time where there are so many
+        int q = tid;
+        if constexpr (V <= 2)
+            for (; q + 7 * NT < R * S; q += 8 * NT) pieces(q, std::integral_constant<int, 8>{});
+        for (; q < R * S; q += NT) pieces(q, std::integral_constant<int, 1>{});
     }
     __syncthreads();
 
     // the batches are dealt to the row groups of all the table's parts
-    const int nb_all = rs[R] / K, g0 = part_i * NG, gg_all = NG * a.parts;
-    const int lo = nb_all / gg_all, extra = nb_all - lo * gg_all;
+    const int nb_all = rs[R] / K, g0 = part_i * NG, gg_all = whole ? NG : NG * a.parts;
+    int lo = nb_all / NG;
+    if (!whole) lo = nb_all / gg_all;
+    const int extra = nb_all - lo * gg_all;
     const int b_begin = (g0 + g) * lo + min(g0 + g, extra), b_end = b_begin + lo + (g0 + g < extra ? 1 : 0);
     int cur = -1;  // row being summed
     float acc[V];
@@ -2449,22 +2469,33 @@ BackwardPlan plan_backward(const Dims &d, int ste_mode, bool lean) {
     // (in the LUT's element type)
     p.rows_dots_rs_off = (d.rows * rows_chunk * esize + 15) & ~15;
     p.rows_dots_part_off = (p.rows_dots_rs_off + (d.rows + 1) * 4 + 15) & ~15;
+    // workgroups of 512 threads where two fit a CU and there are enough: with
+    // several parts, or more units than 1024-thread workgroups are in flight
+    // (one a CU, two with the registers of one column per lane): 200 units of
+    // 500 items, 33 columns 10.6 us, of 1024 threads 8.9. Parts of a (table,
+    // chunk) where the units alone leave a quarter of the GPU's workgroup slots
+    // empty: enough for two rounds, at least four batches a row group
+    auto dots_part_lds = [&](int threads) { return threads / p.rows_slices * 2 * rows_chunk * 4; };
+    const int wide_lds = p.rows_dots_part_off + dots_part_lds(kRowsThreads) + kRowsThreads * 16;
+    const int wide_slots = kCus * (p.rows_vec == 1 && wide_lds <= kRowsSmallLds ? 2 : 1);
     for (p.rows_dots_threads = kRowsSmall;; p.rows_dots_threads = kRowsThreads) {
-        p.rows_dots_ring_off = p.rows_dots_part_off + (p.rows_dots_threads / p.rows_slices) * 2 * rows_chunk * 4;
+        p.rows_dots_ring_off = p.rows_dots_part_off + dots_part_lds(p.rows_dots_threads);
         p.rows_lds_dots_bytes = p.rows_dots_ring_off + p.rows_dots_threads * 16;
-        if (p.rows_dots_threads == kRowsThreads || p.rows_lds_dots_bytes <= kRowsSmallLds) break;
-    }
-    // parts of a (table, chunk), where the units alone leave a quarter of the
-    // GPU's workgroup slots empty: enough for two rounds, at least four batches
-    // a row group
-    {
+        const bool small = p.rows_dots_threads == kRowsSmall;
         const long long units = static_cast<long long>(d.tables) * p.rows_chunks;
-        const int slots = kCus * (p.rows_dots_threads == kRowsSmall ? 2 : 1);
+        const int slots = kCus * (small ? 2 : 1);
         long long parts = units > 0 && units * 4 < slots * 3ll ? (2 * slots + units - 1) / units : 1;
         const long long most = d.items / (4ll * p.rows_batch * (p.rows_dots_threads / p.rows_slices));
         if (parts > most) parts = most;
+        // (one round where a part would walk little beside the LUT chunk it stages,
+        // four round trips of pieces to a batch: 150 tables of 256 rows, 33 columns,
+        // 1500 items 37.7 us in five parts, 28.1 in three)
+        const long long staged = static_cast<long long>(d.rows) * p.rows_slices / p.rows_dots_threads / 4;
+        if (units * parts > slots && parts * staged * p.rows_batch * (p.rows_dots_threads / p.rows_slices) > d.items)
+            parts = slots / units;
         if (parts > kRowsMaxParts) parts = kRowsMaxParts;
         p.rows_parts = parts < 1 || lean ? 1 : static_cast<int>(parts);
+        if (!small || (p.rows_lds_dots_bytes <= kRowsSmallLds && (p.rows_parts > 1 || units > wide_slots))) break;
     }
     // the neighbour row fits below the item offset (a multiple of P * 4 bytes)
     p.rows_nb_pack = rows_chunk * 4 >= d.rows;
