@@ -140,6 +140,9 @@ def test_fused_flag_without_workspace(i, o, t, c, b):
         (32, 33, 6, 7, 70, "f32"),     # the LUT chunk staged eight pieces at a time, 128 rows
         (32, 65, 4, 8, 70, "f16"),     # 256 rows, two chunks
         (32, 33, 150, 8, 1500, "f32"), # three parts: one round of workgroups
+        (16, 1030, 3, 3, 968, "f32"),  # reduce kernel: at most 1024 slots, 17 chunks
+        (16, 1030, 3, 3, 969, "f32"),  # more
+        (16, 33, 5, 2, 900, "f32"),    # at most 1024 slots in three parts
         (16, 35, 2, 5, 3000, "f32"),   # one-column pieces of G over many copy workgroups
     ],
 )

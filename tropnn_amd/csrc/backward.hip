@@ -1070,17 +1070,25 @@ __device__ __forceinline__ void merge_part_rows(const ReduceArgs &a, int t) {
     }
 }
 
+// MERGE: with merge_part_rows' workgroups (a kernel of its own: beside their
+// barriers and atomics the compiler turns the uniform loads into vector ones).
+// FEW: at most kReduceThreads slots, one a thread, more chunks of it in flight
+// (a kernel of its own too: 500 tables of 300 items 4.3 us, 5.8 beside the other
+// walk and its registers; 32 items of 64 chunks 7.0 us, 13.1 with four slots).
+template <bool MERGE, bool FEW>
 __global__ __launch_bounds__(kReduceThreads) void pairwise_bwd_reduce_kernel(ReduceArgs a) {
-    constexpr int kWaves = kReduceThreads / kWave, kU = 4;
+    constexpr int kWaves = kReduceThreads / kWave;
+    constexpr int kU = FEW ? 1 : 4, kD = FEW ? 8 : 4;  // slots of a thread, chunks of each in flight
     __shared__ float tp[kWaves * 8];
     // with `stage`, the table's {gu, r} records gather in LDS (in item order)
     // and leave as whole lines after the walk, instead of as scattered
     // 8-byte stores
     extern __shared__ __align__(16) uint64_t gstage[];  // [items]
-    if (static_cast<int>(blockIdx.x) >= a.tables) {  // uniform per workgroup
-        merge_part_rows(a, blockIdx.x - a.tables);
-        return;
-    }
+    if constexpr (MERGE)
+        if (static_cast<int>(blockIdx.x) >= a.tables) {  // uniform per workgroup
+            merge_part_rows(a, blockIdx.x - a.tables);
+            return;
+        }
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint64_t *rec_t = a.rec + static_cast<size_t>(t) * a.items;
@@ -1101,7 +1109,6 @@ __global__ __launch_bounds__(kReduceThreads) void pairwise_bwd_reduce_kernel(Red
         for (int u = 0; u < kU; ++u) dot[u] = 0.f;
         // the slots' dots, kD chunks of each in flight, summed in chunk order
         // (a padding slot's dots are loaded and dropped)
-        constexpr int kD = 4;
         auto sum = [&](int c, auto n) {
             constexpr int N = decltype(n)::value;
             float v[N][kU];
@@ -2892,7 +2899,10 @@ hipError_t launch_backward(const Dims &d, const BackwardPlan &p, const float *gr
         return hipGetLastError();
     }
     ra.stage = ra.gurec != nullptr && d.items <= kReduceStageBytes / 8;
-    if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_REDUCE, pairwise_bwd_reduce_kernel,
+    const bool few = p.sort_slots <= kReduceThreads;
+    const auto reduce = ra.parts > 1 ? (few ? pairwise_bwd_reduce_kernel<true, true> : pairwise_bwd_reduce_kernel<true, false>)
+                                     : (few ? pairwise_bwd_reduce_kernel<false, true> : pairwise_bwd_reduce_kernel<false, false>);
+    if (hipError_t e = launch_kernel(TROPNN_KERNEL_BACKWARD_REDUCE, reduce,
                                      dim3(ra.parts > 1 ? 2 * d.tables : d.tables),
                                      dim3(kReduceThreads), ra.stage ? d.items * 8 : 0, stream, ra);
         e != hipSuccess || grad_x == nullptr)
