@@ -222,7 +222,10 @@ int tropnn_hip_pairwise_backward(int64_t items, int64_t in_features, int64_t out
  * TROPNN_NOALLOC_WORKSPACE_BYTES that the library holds, one per GPU, from
  * the first call on that GPU until the process ends. The call allocates
  * nothing. A shape whose workspace (tropnn_hip_pairwise_backward_workspace_size)
- * is larger fails with TROPNN_ERR_UNSUPPORTED before any launch. Every call
+ * is larger runs a backward that keeps less in it (no tables or rows shared
+ * between workgroups, full STE by items: slower at large batches, gradients
+ * equal to f32 rounding, its sums in another order); where that one does not
+ * fit either, the call fails with TROPNN_ERR_UNSUPPORTED before any launch. Every call
  * on one GPU shares that GPU's buffer: calls that overlap on one GPU (other
  * streams, other threads, without ordering between them) race on it and give
  * wrong gradients; serialise them. The buffer needs no clearing between calls.
