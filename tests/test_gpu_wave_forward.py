@@ -161,6 +161,12 @@ def test_wave_shapes_with_lut_or_output_off_16_bytes(lut_dtype, o, lut_off, out_
         (20, 98, 70, 6, 4100, "f16"),    # 196 of 256 bytes, f16 rows on 4-byte boundaries
         (20, 449, 40, 8, 2100, "f32"),   # two column tiles, 772 bytes of the second
         (20, 200, 160, 7, 2051, "f32"),  # whole 16-byte pieces that end inside the tile
+        (20, 227, 11, 5, 12288, "f32"),  # the fewest tables of many items, one-tile rows
+        (20, 227, 10, 5, 12288, "f32"),  # too few: the multi-item kernel
+        (20, 227, 10, 5, 12287, "f32"),  # fewer items
+        (20, 453, 11, 5, 4095, "f32"),   # the fewest tables of two-tile rows, the most items
+        (20, 453, 11, 5, 4096, "f32"),   # too many
+        (20, 453, 17, 5, 4096, "f32"),   # any number from 17 tables on
     ],
 )
 def test_wave_forward_rows_that_fill_no_power_of_two(i, o, t, c, b, lut_dtype):

@@ -428,6 +428,7 @@ constexpr int kWaveThreads = 256;
 constexpr int kWaveWaves = kWaveThreads / kWave;
 constexpr int kWaveBlock = 16;    // tables per block, at most (the plan's per_wave)
 constexpr int kWaveMinItems = 2048;
+constexpr int kWaveRaggedItems = 4096, kWaveRaggedMany = 12288;
 constexpr int kWaveMinWaves = 1024;  // below, the one-item and multi-item kernels spread the work wider
 constexpr int kWaveRing = 2;         // blocks of row loads in flight (3 and 4 measured slower)
 
@@ -1089,6 +1090,22 @@ ForwardPlan plan_forward(const Dims &d, bool rows16) {
     //    against 16.7, 3000 17.7 against 18.0, 8192 44 -> 42; 200 f16 columns,
     //    2051 items 13.6 against 14.2, 4096 24 -> 16; from a larger LUT always
     //    (300 tables of 64 rows, 256 f32 columns, 2051 items 84 -> 53).
+    // Rows that fill no power of two leave lanes idle and cross lines, so those
+    // need more (500 shapes of 500 to 40000 items, against the other kernels):
+    //  - 40 tables against the one-item kernel with 16-byte loads (736 f32
+    //    columns, 18 tables, 5170 items 24 against 36; 508, 33 tables, 3018 items
+    //    19.5 against 25; 472 f16 columns, 46 tables, 10358 items 41 -> 37);
+    //  - 17 against the multi-item kernel, which has so few tables' rows in flight
+    //    at once (454 columns, 14 tables, 5949 items 18 against 24; 196 f16
+    //    columns, 13 tables, 36797 items 53 against 67); with f32 rows of one
+    //    tile, or under 4096 items of fewer than 256 rows, 11 (227, 13 tables,
+    //    28173 items 71 -> 53; 661, 12 tables, 2335 items 25 -> 17), of one tile
+    //    and under 12288 items any (107, 9 tables, 5161 items 12.3 -> 8.9; 110, 9
+    //    tables, 34696 items 23 against 32);
+    //  - fewer than 12288 items over up to 64 tables of 256 rows past an XCD's L2
+    //    (457 columns, 46 tables, 22328 items 148 against 170; 118, 39 tables,
+    //    23335 items 46 against 54; 579, 24 tables, 3075 items 31 -> 28; 119, 177
+    //    tables, 17876 items 223 -> 138).
     p.wave = false;
     {
         const int row_bytes = d.out_f * esize;
@@ -1098,7 +1115,15 @@ ForwardPlan plan_forward(const Dims &d, bool rows16) {
         const bool vec16 = p.vec * esize == 16, in_l2 = static_cast<long long>(row_bytes) * d.tables * d.rows <= (4ll << 20);
         const bool enough = d.items >= kWaveMinItems ? !(vec16 && in_l2) || elements >= (esize == 4 ? 60e6 : 40e6)
                                                      : !vec16 && elements >= 25e6;
-        if (rows16 && enough && (d.items + ipw - 1) / ipw >= kWaveMinWaves && tile > 0 && d.in_f <= 16384) {
+        auto pays = [&] {
+            if ((row_bytes & (row_bytes - 1)) == 0) return true;
+            if (vec16) return d.tables >= 40;
+            if (d.rows == 256 && !in_l2 && d.items >= kWaveRaggedMany && d.tables <= 64) return false;
+            return d.tables > 16 ||
+                   (esize == 4 && (row_bytes <= 1024 ? d.tables > 10 || d.items < kWaveRaggedMany
+                                                     : d.tables > 10 && d.items < kWaveRaggedItems && d.rows < 256));
+        };
+        if (rows16 && enough && pays() && (d.items + ipw - 1) / ipw >= kWaveMinWaves && tile > 0 && d.in_f <= 16384) {
             const int w16 = (d.tables + kWaveBlock - 1) / kWaveBlock;
             const int per16 = (d.tables + w16 - 1) / w16;
             const int lpr = tile / 16;
