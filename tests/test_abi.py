@@ -307,6 +307,13 @@ def test_forward_workspace(lib):
     assert ws(2048, 256, 512, 512, 6, ph.LUT_F16) == 0  # 71 us in one launch, 118 us staged
     assert ws(4095, 1024, 128, 512, 8, ph.LUT_F16) == 0  # 78 us against 269 us
     assert ws(4096, 1024, 128, 512, 8, ph.LUT_F16) > 0  # for training only (streamed: 452 us)
+    # rows off 16-byte boundaries: both sides of the closer estimates
+    assert ws(37702, 70, 346, 9, 6, ph.LUT_F16) == 0  # 52 us plain, 83 staged
+    assert ws(22328, 28, 457, 46, 8, ph.LUT_F32) == 0  # 148 against 250
+    assert ws(4421, 88, 563, 72, 7, ph.LUT_F32) == 0  # 82 against 106
+    assert ws(37930, 33, 619, 50, 7, ph.LUT_F32) > 0  # 339 against 195
+    assert ws(10762, 27, 515, 290, 7, ph.LUT_F16) > 0  # 1102 against 437
+    assert ws(33418, 450, 259, 15, 4, ph.LUT_F16) > 0  # 132 against 68
     assert ws(8192, 20000, 128, 136, 6, ph.LUT_F32) == 0  # input rows beyond a workgroup's LDS
     assert ws(8192, 128, 128, 136, 9, ph.LUT_F32) == 0 and "comparisons" in _err(lib)
     fwd = lib.tropnn_hip_pairwise_forward_ws
@@ -320,7 +327,8 @@ def test_forward_workspace(lib):
 
 def test_forward_planning_stays_short(lib):
     """Narrow rows over very large batches: the launch shape is searched over
-    the distinct block sizes only, and the size query does not search. A call
+    the distinct block sizes only, and the size query does not search where rows are
+    whole 16-byte pieces. A call
     refused for its workspace's size plans in full: 16 us when every count of
     blocks was tried, 1 to 2 us now (the least of many, so that other load on
     the machine does not count)."""

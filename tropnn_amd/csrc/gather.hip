@@ -661,6 +661,46 @@ hipError_t launch_stream_words_ipt(const StreamWordsArgs &s, const GatherPlan &p
     }
 }
 
+// Rows off 16-byte boundaries are staged and stored in smaller pieces, which
+// plan_gather's first estimate leaves out. Of those both sides are estimated
+// closer, from fits to 500 shapes of 500 to 40000 items, 8 to 300 tables (the
+// staged side 0.72 to 1.23 of the measured time in nine of ten). Staged although
+// slower before: 346 f16 columns, 9 tables of 64 rows, 37702 items 83 us against
+// 52 plain; 457 f32 columns, 46 tables of 256, 22328 items 250 against 148; 563,
+// 72 of 128, 4421 items 106 against 82; 1073 f16 columns, 112 of 256, 7146 items
+// 525 against 287. Kept: 619 f32 columns, 50 of 128, 37930 items 339 -> 195; 515
+// f16 columns, 290 of 128, 10762 items 1102 -> 437.
+
+// Staged: `staged` rows a workgroup slot stages in turn, in cycles of a CU
+// (staged_cu) by the piece the rows' alignment leaves, more per 4-byte piece and
+// less where many rows come in turn past the caches; the sums' cycles; the
+// output's and the input's MB.
+double slice_us(const Dims &d, int row_bytes, double staged, double staged_cu, double summed) {
+    const bool f16 = d.lut_dtype == TROPNN_LUT_F16;
+    double row = row_bytes % 8 == 0 ? 2.75 : row_bytes % 4 == 0 ? 3.2 : 8.1;
+    if (row_bytes % 8 != 0 && staged > 16000.) row += 2.6;
+    const double kcycles = 1.0 / 2400.0;  // us a cycle
+    return 8.6 + kcycles * (row * staged_cu + (f16 ? 1.24 : 0.55) * summed) +
+           4e-6 * d.items * (d.out_f * (d.out_f % 4 == 0 ? 0.38 : 1.23) + d.in_f * 0.19);
+}
+
+// Plain: a start, thousands of gathered elements per us and us per MB of output,
+// by the lane's load (the wave-item kernel's is 16 bytes) and whether an XCD's L2
+// holds the LUT.
+double plain_slice_us(const Dims &d, double elements, bool in_l2) {
+    struct Rate {
+        double start, rate, out;
+    };
+    constexpr Rate kF32[3][2] = {{{6.2, 2096, 0}, {5.6, 2629, 0.29}}, {{7.9, 2731, 0}, {5.2, 2979, 0.45}}, {{11.7, 5203, 0.85}, {5.3, 7238, 1.24}}};
+    constexpr Rate kF16[4][2] = {{{15.7, 2528, 0}, {9.7, 2826, 0.52}}, {{12.5, 3779, 0.13}, {7.6, 4734, 0.48}}, {{12, 3763, 0}, {12.8, 6281, 0}}, {{21.8, 10182, 0.43}, {10, 12810, 0.54}}};
+    const ForwardPlan f = plan_forward(d);
+    const bool f16 = d.lut_dtype == TROPNN_LUT_F16;
+    const int vec = std::min(f.vec, f16 ? 4 : 2);  // (16-byte loads: rows of whole 16 bytes)
+    const Rate r = f16 ? kF16[f.wave ? 3 : vec == 4 ? 2 : vec - 1][in_l2] : kF32[f.wave ? 2 : vec - 1][in_l2];
+    const double us = r.start + elements / r.rate + 4e-6 * d.items * d.out_f * r.out;
+    return f.wave ? 1.3 * us : us;  // (the wave-item kernel's fits are the looser ones)
+}
+
 }  // namespace
 
 GatherPlan plan_gather(const Dims &d, bool size_only) {
@@ -776,7 +816,8 @@ GatherPlan plan_gather(const Dims &d, bool size_only) {
         p.stages = (p.blocks + p.stage_blocks - 1) / p.stage_blocks;
         p.lds_bytes = lds_for(p.stage_blocks);
         if (p.lds_bytes > kMaxLdsBytes) return p;
-        if (size_only) {
+        const bool whole = row_bytes % kSliceBytes == 0;
+        if (size_only && whole) {
             p.ok = true;
             return p;
         }
@@ -786,7 +827,7 @@ GatherPlan plan_gather(const Dims &d, bool size_only) {
         // item blocks: the least estimated time, in cycles of one CU: a
         // staged LDS row costs about one (its line's request), a wave's read
         // of 16-byte rows about 12
-        double best = 0;
+        double best = 0, staged = 0, summed = 0;
         const int slots = kGatherCus * per_cu;
         const int max_blk = std::max(1, std::min((d.items + kWave - 1) / kWave, 4 * slots / p.slices + 1));
         for (int nblk = 1; nblk <= max_blk;) {
@@ -801,14 +842,19 @@ GatherPlan plan_gather(const Dims &d, bool size_only) {
             const long long wgs = static_cast<long long>((d.items + bi - 1) / bi) * p.slices;
             const double stage = 1.0 * d.tables * d.rows * (p.stages > 1 ? passes : 1) + 3000.0;
             const double sum = 12.0 * passes * p.slice_ipt * (thr / kWave) * d.tables;
-            const double cost = static_cast<double>((wgs + slots - 1) / slots) * (stage + sum) * per_cu;
+            const double rounds = static_cast<double>((wgs + slots - 1) / slots);
+            const double cost = rounds * (stage + sum) * per_cu;
             if (best == 0 || cost < best) {
                 best = cost;
                 p.block_items = bi;
                 p.threads = thr;
                 p.wgs = static_cast<int>(wgs);
+                staged = rounds * (stage - 3000.0);
+                summed = rounds * sum * per_cu;
             }
         }
+        // (at most 16 rows a table are staged in no time, and the fits miss those)
+        if (!whole && d.rows > 16 && slice_us(d, static_cast<int>(row_bytes), staged, staged * per_cu, summed) > plain_slice_us(d, elements, in_l2)) return p;
     }
     p.ok = true;
     return p;
